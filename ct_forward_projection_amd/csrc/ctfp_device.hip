@@ -540,37 +540,15 @@ struct MarchArgs {
     // through it
     const uint8_t *odist;
     // ray tile: wavefronts of (1 << wu_log2) x (64 >> wu_log2) pixels,
-    // (1 << bu_log2) x (4 >> bu_log2) wavefronts per workgroup
+    // (1 << bu_log2) x (4 >> bu_log2) wavefronts per workgroup; order of a
+    // wavefront's lanes (tile_lane)
     int32_t wu_log2, bu_log2;
+    int32_t pass_order;
 };
 
 constexpr int kBlock = 256; // 4 wavefronts per workgroup
 // Zero rows after the last active bin of the spectral weight table.
 constexpr int kWeightPadBins = 8;
-
-template <int M>
-__device__ __forceinline__ void load_vox(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff,
-                                         float (&c)[M])
-{
-    if constexpr (M == 1) {
-        c[0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
-    } else if constexpr (M == 2) {
-        auto v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0);
-        c[0] = __uint_as_float(v[0]);
-        c[1] = __uint_as_float(v[1]);
-    } else if constexpr (M == 3) {
-        auto v = __builtin_amdgcn_raw_buffer_load_b96(r, voff, soff, 0);
-        c[0] = __uint_as_float(v[0]);
-        c[1] = __uint_as_float(v[1]);
-        c[2] = __uint_as_float(v[2]);
-    } else {
-        auto v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
-        c[0] = __uint_as_float(v[0]);
-        c[1] = __uint_as_float(v[1]);
-        c[2] = __uint_as_float(v[2]);
-        c[3] = __uint_as_float(v[3]);
-    }
-}
 
 // Support interval of index s + k*d inside (a, b): intersect into [lo, hi].
 // (-1, n) is the support of a volume of n voxels: a sample outside it has no
@@ -623,6 +601,24 @@ struct RayLine {
     double sa, sb, sc; // source (t = 0)
     double da, db, dc; // d(index)/dt
 };
+// The source of view vw in index space: every ray of the view starts there.
+__device__ __forceinline__ void ray_source(const MarchArgs &P, int vw, double &sa, double &sb, double &sc)
+{
+#pragma clang fp contract(off)
+    const double2 cs = P.view_cs[vw];
+    if (!P.focal) {
+        sa = (P.half_x - P.sod * cs.x) * P.inv_px;
+        sb = (P.half_y + P.sod * cs.y) * P.inv_py;
+        sc = P.half_z * P.inv_pz;
+        return;
+    }
+    // (-SOD, su, sv) rotated like every sample
+    const double2 f = P.focal[vw];
+    sa = (P.half_x - P.sod * cs.x - f.x * cs.y) * P.inv_px;
+    sb = (P.half_y + P.sod * cs.y - f.x * cs.x) * P.inv_py;
+    sc = (P.half_z - f.y) * P.inv_pz;
+}
+
 __device__ __forceinline__ RayLine ray_line(const MarchArgs &P, int u, int v, int vw)
 {
 #pragma clang fp contract(off)
@@ -640,13 +636,11 @@ __device__ __forceinline__ RayLine ray_line(const MarchArgs &P, int u, int v, in
     double dX = cg * cb, dY = cg * sb, dZ = sg;
     // transformKernel (CBCTPolyProjGPU.cu:1915-1917) is affine in t.
     RayLine L;
+    ray_source(P, vw, L.sa, L.sb, L.sc);
     if (!P.focal) {
         L.da = (dX * cs.x - dY * cs.y) * P.inv_px;
         L.db = -(dX * cs.y + dY * cs.x) * P.inv_py;
         L.dc = -dZ * P.inv_pz;
-        L.sa = (P.half_x - P.sod * cs.x) * P.inv_px;
-        L.sb = (P.half_y + P.sod * cs.y) * P.inv_py;
-        L.sc = P.half_z * P.inv_pz;
         return L;
     }
     // Focal spot: the source moves to (-SOD, su, sv) in its frame and the ray
@@ -659,10 +653,6 @@ __device__ __forceinline__ RayLine ray_line(const MarchArgs &P, int u, int v, in
     L.da = (ex * cs.x - ey * cs.y) * P.inv_px;
     L.db = -(ex * cs.y + ey * cs.x) * P.inv_py;
     L.dc = -ez * P.inv_pz;
-    // source (-SOD, su, sv) rotated like every sample
-    L.sa = (P.half_x - P.sod * cs.x - f.x * cs.y) * P.inv_px;
-    L.sb = (P.half_y + P.sod * cs.y - f.x * cs.x) * P.inv_py;
-    L.sc = (P.half_z - f.y) * P.inv_pz;
     return L;
 }
 
@@ -874,21 +864,6 @@ __device__ __forceinline__ void load_glob(const char *p, uint32_t (&c)[M])
     for (int m = 0; m < M; m++) c[m] = q[m];
 }
 
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-typedef short bf16x2_t __attribute__((ext_vector_type(2)));
-
-// acc += w.x * lo(d) + w.y * hi(d), FP32 accumulate (v_dot2_f32_f16 / _bf16).
-template <int ST>
-__device__ __forceinline__ float dot2_acc(uint32_t w, uint32_t d, float acc)
-{
-    if constexpr (ST == kStF16)
-        return __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, w), __builtin_bit_cast(half2_t, d), acc,
-                                      false);
-    else
-        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w),
-                                               __builtin_bit_cast(bf16x2_t, d), acc, false);
-}
-
 typedef __bf16 bf16x2_v __attribute__((ext_vector_type(2)));
 typedef float f32x2_v __attribute__((ext_vector_type(2)));
 
@@ -1019,106 +994,159 @@ __device__ __forceinline__ void segment_box(const Anchor &A, int i0, int i1, int
     hi[2] = max(hi[2], A.ic + max(a.z, b.z) + 1);
 }
 
-// Trilinear accumulation of one sample into the M per-material sums from
-// 8 corners (FP32 voxels) or 4 rows of x-pairs (16-bit).  `fetch(row, out)`
-// returns the M dwords at corner row `row` (0: y0z0, 1: y1z0, 2: y0z1,
-// 3: y1z1) and, for FP32, `fetch(row + 4, out)` the x+1 corner.
-template <int M, int ST, typename Fetch>
-__device__ __forceinline__ void accumulate(const Cell &c, Fetch fetch, float (&acc)[M])
+// acc += w.x * lo(d) + w.y * hi(d), FP32 accumulate (v_dot2_f32_f16 / _bf16).
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef short bf16x2_t __attribute__((ext_vector_type(2)));
+template <int ST>
+__device__ __forceinline__ float dot2_acc(uint32_t w, uint32_t d, float acc)
 {
-    if constexpr (ST == kStF32) {
-        const float bx = 1.0f - c.ax, by = 1.0f - c.ay, bz = 1.0f - c.az;
-        uint32_t d[8][M];
-#pragma unroll
-        for (int r = 0; r < 8; r++) fetch(r, d[r]);
-        const float wr[4] = {by * bz, c.ay * bz, by * c.az, c.ay * c.az};
-#pragma unroll
-        for (int m = 0; m < M; m++) {
-            float a = acc[m];
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                a = fmaf(bx * wr[r], __uint_as_float(d[r][m]), a);
-                a = fmaf(c.ax * wr[r], __uint_as_float(d[r + 4][m]), a);
-            }
-            acc[m] = a;
-        }
-    } else {
-        uint32_t d[4][M];
-#pragma unroll
-        for (int r = 0; r < 4; r++) fetch(r, d[r]);
-        // (y, z) row weights; (1 - ay) * b as the fma b - ay * b
-        const float bz = 1.0f - c.az;
-        const float w00 = fmaf(-c.ay, bz, bz), w10 = c.ay * bz, w01 = fmaf(-c.ay, c.az, c.az),
-                    w11 = c.ay * c.az;
-        const uint32_t p[4] = {x_pair<ST>(w00, c.ax), x_pair<ST>(w10, c.ax), x_pair<ST>(w01, c.ax),
-                               x_pair<ST>(w11, c.ax)};
-#pragma unroll
-        for (int m = 0; m < M; m++) {
-            float a = acc[m];
-#pragma unroll
-            for (int r = 0; r < 4; r++) a = dot2_acc<ST>(p[r], d[r][m], a);
-            acc[m] = a;
-        }
-    }
+    if constexpr (ST == kStF16)
+        return __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, w), __builtin_bit_cast(half2_t, d), acc,
+                                      false);
+    else
+        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w),
+                                               __builtin_bit_cast(bf16x2_t, d), acc, false);
 }
 
-// Global-memory gather of one sample (raw buffer loads; one VGPR offset).
-template <int M, int ST, bool W>
-__device__ __forceinline__ void accumulate_global(__amdgpu_buffer_rsrc_t rsrc, const char *vol, const Cell &c,
+// Trilinear weights of one plane (z0 or z1) of a sample, in the order its
+// corners are added: the rows y0, y1, each as the corners x0, x1 (FP32) or as
+// one x-pair (16-bit).  (Weighting a plane by (x, y) first and by z after
+// would save 2 to 7 instructions a sample, but rounds every line integral
+// differently.)
+template <int ST> struct PlaneWeights {
+    float w[4];
+};
+template <> struct PlaneWeights<kStF16> {
+    uint32_t w[2];
+};
+template <> struct PlaneWeights<kStBF16> {
+    uint32_t w[2];
+};
+template <int ST> __device__ __forceinline__ PlaneWeights<ST> plane_weights(const Cell &c, int z)
+{
+    PlaneWeights<ST> k;
+    const float wz = z ? c.az : 1.0f - c.az;
+    if constexpr (ST == kStF32) {
+        const float bx = 1.0f - c.ax, by = 1.0f - c.ay;
+        const float w0 = by * wz, w1 = c.ay * wz;
+        k.w[0] = bx * w0;
+        k.w[1] = c.ax * w0;
+        k.w[2] = bx * w1;
+        k.w[3] = c.ax * w1;
+    } else {
+        // (1 - ay) * wz as the fma wz - ay * wz
+        k.w[0] = x_pair<ST>(fmaf(-c.ay, wz, wz), c.ax);
+        k.w[1] = x_pair<ST>(c.ay * wz, c.ax);
+    }
+    return k;
+}
+
+// Corner cells of one plane: the four corners in the order of the weights, or
+// the two x-pair rows of 16-bit storage.
+template <int ST> constexpr int kPlaneCells = ST == kStF32 ? 4 : 2;
+
+// Adds plane z of sample c to the M sums.  `cell(i, m)` is dword m of the
+// plane's cell i.
+template <int M, int ST, typename F>
+__device__ __forceinline__ void add_plane(const Cell &c, int z, F cell, float (&acc)[M])
+{
+    const PlaneWeights<ST> k = plane_weights<ST>(c, z);
+#pragma unroll
+    for (int m = 0; m < M; m++)
+#pragma unroll
+        for (int i = 0; i < kPlaneCells<ST>; i++) {
+            if constexpr (ST == kStF32)
+                acc[m] = fmaf(k.w[i], __uint_as_float(cell(i, m)), acc[m]);
+            else
+                acc[m] = dot2_acc<ST>(k.w[i], cell(i, m), acc[m]);
+        }
+}
+
+// Global-memory gather of N samples, all their loads in flight together.
+template <int M, int ST, bool W, int N>
+__device__ __forceinline__ void accumulate_global(__amdgpu_buffer_rsrc_t rsrc, const char *vol, const Cell (&c)[N],
                                                   uint32_t oy, uint32_t oz, float (&acc)[M])
 {
     constexpr uint32_t CB = 4u * M;
-    // Byte offset with full-rate 24-bit multiply-adds: the masks (no-ops on
-    // the clamped cells) tell the compiler every factor is < 2^24; the
-    // strides are < 2^24 and the offset < 2^32 (checked at allocation).
-    const uint32_t xi = (uint32_t)(c.x + kVoxPadLo) & 0xFFFFFu;
-    const uint32_t yi = (uint32_t)(c.y + kVoxPadLo) & 0xFFFFFu;
-    const uint32_t zi = (uint32_t)(c.z + kVoxPadLo) & 0xFFFFFu;
-    const uint32_t soff[4] = {0u, oy, oz, oy + oz};
-    if constexpr (W) {
-        // a volume of 4 GiB or more: a 64-bit z offset; within a slice
-        // (< 16 MiB) the y and x offsets stay 32-bit
-        const char *p = vol + ((uint64_t)zi * oz + (yi * oy + xi * CB));
-        accumulate<M, ST>(c, [&](int r, uint32_t(&out)[M]) {
-            load_glob<M>(p + soff[r & 3] + (r < 4 ? 0u : CB), out);
-        }, acc);
-    } else {
-        const uint32_t voff = zi * oz + (yi * oy + xi * CB);
-        accumulate<M, ST>(c, [&](int r, uint32_t(&out)[M]) {
-            load_raw<M>(rsrc, r < 4 ? voff : voff + CB, soff[r & 3], out);
-        }, acc);
+    constexpr int NP = kPlaneCells<ST>;
+    uint32_t d[N][2][NP][M];
+    // cell i of a plane: x + (i & 1), y + (i >> 1) (FP32), or y + i (x-pairs)
+    auto xo = [](int i) { return ST == kStF32 && (i & 1) ? CB : 0u; };
+    auto yo = [&](int i) { return (ST == kStF32 ? i >> 1 : i) ? oy : 0u; };
+#pragma unroll
+    for (int n = 0; n < N; n++) {
+        // Byte offset with full-rate 24-bit multiply-adds: the masks (no-ops
+        // on the clamped cells) tell the compiler every factor is < 2^24; the
+        // strides are < 2^24 and the offset < 2^32 (checked at allocation).
+        const uint32_t xi = (uint32_t)(c[n].x + kVoxPadLo) & 0xFFFFFu;
+        const uint32_t yi = (uint32_t)(c[n].y + kVoxPadLo) & 0xFFFFFu;
+        const uint32_t zi = (uint32_t)(c[n].z + kVoxPadLo) & 0xFFFFFu;
+        if constexpr (W) {
+            // a volume of 4 GiB or more: a 64-bit z offset; within a slice
+            // (< 16 MiB) the y and x offsets stay 32-bit
+            const char *p = vol + ((uint64_t)zi * oz + (yi * oy + xi * CB));
+#pragma unroll
+            for (int i = 0; i < 2 * NP; i++)
+                load_glob<M>(p + ((i < NP ? 0u : oz) + yo(i % NP) + xo(i % NP)), d[n][i / NP][i % NP]);
+        } else {
+            const uint32_t voff = zi * oz + (yi * oy + xi * CB);
+#pragma unroll
+            for (int i = 0; i < 2 * NP; i++)
+                load_raw<M>(rsrc, voff + xo(i % NP), (i < NP ? 0u : oz) + yo(i % NP), d[n][i / NP][i % NP]);
+        }
     }
+#pragma unroll
+    for (int n = 0; n < N; n++) {
+        add_plane<M, ST>(c[n], 0, [&](int i, int m) { return d[n][0][i][m]; }, acc);
+        add_plane<M, ST>(c[n], 1, [&](int i, int m) { return d[n][1][i][m]; }, acc);
+    }
+}
+
+// Samples [i, i1) after anchor A, gathered from global memory kN at a time
+// (a chunk's worth of loads per round trip: the gather is bound by latency
+// and, with coarse detectors, by the L2).
+template <int M, int ST, bool W, int kN>
+__device__ __forceinline__ void gather_segment(__amdgpu_buffer_rsrc_t rsrc, const char *vol, const Anchor &A, int i,
+                                               int i1, int nx, int ny, int nz, uint32_t oy, uint32_t oz, float (&acc)[M])
+{
+    float fi = (float)i;
+    if constexpr (kN > 1)
+        for (; i + kN <= i1; i += kN, fi += (float)kN) {
+            Cell c[kN];
+#pragma unroll
+            for (int n = 0; n < kN; n++) c[n] = absolute_cell(A, offset_cell(A, fi + (float)n), nx, ny, nz);
+            accumulate_global<M, ST, W, kN>(rsrc, vol, c, oy, oz, acc);
+        }
+    for (; i < i1; i++, fi += 1.0f) {
+        const Cell c[1] = {absolute_cell(A, offset_cell(A, fi), nx, ny, nz)};
+        accumulate_global<M, ST, W, 1>(rsrc, vol, c, oy, oz, acc);
+    }
+}
+// Samples in flight with at most `regs` registers of corners (1, 2, 4 or 8).
+constexpr int gather_samples(int M, int st, int regs)
+{
+    const int one = (st == kStF32 ? 8 : 4) * M;
+    return regs >= 8 * one ? 8 : regs >= 4 * one ? 4 : regs >= 2 * one ? 2 : 1;
 }
 
 // Bytes of one staged cell in LDS: M dwords, three padded to four so every
 // cell read is one aligned ds_read.
 template <int M> constexpr uint32_t lds_cell_bytes() { return M == 3 ? 16u : 4u * M; }
 
-template <int M>
-__device__ __forceinline__ void lds_read(const char *lds, uint32_t off, uint32_t (&c)[M])
-{
-    if constexpr (M == 1) {
-        c[0] = *(const uint32_t *)(lds + off);
-    } else if constexpr (M == 2) {
-        uint2 v = *(const uint2 *)(lds + off);
-        c[0] = v.x;
-        c[1] = v.y;
-    } else {
-        // All 16 bytes, padding included: ds_read_b128 serves a wavefront
-        // in fewer LDS cycles than ds_read_b96 (1.44x the lane rate on
-        // gfx950).  The volatile access keeps the compiler from narrowing
-        // the load to the three dwords that are used; the explicit LDS
-        // address space keeps it a ds_read (volatile accesses are not
-        // moved from generic to LDS addressing by the compiler).
-        typedef uint32_t u32x4_v __attribute__((ext_vector_type(4)));
-        typedef const volatile __attribute__((address_space(3))) u32x4_v lds_u32x4;
-        const u32x4_v v = *(lds_u32x4 *)(lds + off);
-        c[0] = v.x;
-        c[1] = v.y;
-        c[2] = v.z;
-        if constexpr (M == 4) c[3] = v.w;
-    }
-}
+// One staged cell as it is read from LDS: all four dwords of a three-channel
+// cell, pad included (ds_read_b128 serves a wavefront in fewer LDS cycles
+// than ds_read_b96: 1.44x the lane rate on gfx950).
+typedef uint32_t u32x2_v __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4_v __attribute__((ext_vector_type(4)));
+template <int M> struct CellWords {
+    typedef u32x4_v type;
+};
+template <> struct CellWords<1> {
+    typedef uint32_t type;
+};
+template <> struct CellWords<2> {
+    typedef u32x2_v type;
+};
 
 template <int M>
 __device__ __forceinline__ void lds_write(char *lds, uint32_t off, const uint32_t (&c)[M])
@@ -1128,13 +1156,36 @@ __device__ __forceinline__ void lds_write(char *lds, uint32_t off, const uint32_
     } else if constexpr (M == 2) {
         *(uint2 *)(lds + off) = make_uint2(c[0], c[1]);
     } else if constexpr (M == 3) {
-        *(uint4 *)(lds + off) = make_uint4(c[0], c[1], c[2], 0u);
+        uint4 v; // (the pad dword holds anything)
+        v.x = c[0];
+        v.y = c[1];
+        v.z = c[2];
+        *(uint4 *)(lds + off) = v;
     } else {
         *(uint4 *)(lds + off) = make_uint4(c[0], c[1], c[2], c[3]);
     }
 }
 
-// Ray geometry of the lane's pixel (or an empty range for lanes past the edge).
+// A wavefront's lanes in the order in which a 16-byte LDS read serves them:
+// gfx950 serves such a read 16 lanes at a time, the lanes of groups of four
+// {0, 3, 5, 6} (0-3, 12-15, 20-27), then {1, 2, 4, 7}, then the same of the
+// upper half; lanes of one pass that read different cells collide when the
+// cell indices are equal mod 16.  This index makes each pass's 16 lanes
+// consecutive.
+__device__ __forceinline__ int pass_lane(int lane)
+{
+    const int g = (lane >> 2) & 7;
+    return (lane & 35) | (((g ^ (g >> 1) ^ (g >> 2)) & 1) << 4) | ((g >> 1) << 2);
+}
+
+// Ray geometry of the lane's pixel (or an empty range for lanes past the
+// edge).  For staged marches (pass_order) v runs fastest over the lanes of an
+// LDS pass: neighbours in v cross nearly the same (x, y) cells in successive z
+// planes, whose distance in LDS the staging chooses (box_plane), so a read of
+// 2 x 8 rays takes ~1.1 passes where rows of u took ~1.8 (a model of the
+// sample addresses; the 3 x 512^3 FP16 scan's conflict cycles fell from 52 %
+// to 1.4 % of the LDS's).  Otherwise u runs fastest: neighbours in u often
+// share the volume's cache lines.
 struct TileLane {
     int vw_local, u, v;
     bool active;
@@ -1146,11 +1197,17 @@ __device__ __forceinline__ TileLane tile_lane(const MarchArgs &P, uint32_t logic
     t.vw_local = (int)(logical / tiles);
     const uint32_t q = logical % tiles;
     const int tile_v = (int)(q / P.tiles_u), tile_u = (int)(q % P.tiles_u);
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int wu = P.wu_log2, bu = P.bu_log2;
+    const int wave = threadIdx.x >> 6, wu = P.wu_log2, bu = P.bu_log2;
+    int lane = threadIdx.x & 63;
+    int lu = lane & ((1 << wu) - 1), lv = lane >> wu;
+    if (P.pass_order) {
+        lane = pass_lane(lane);
+        lu = lane >> (6 - wu);
+        lv = lane & ((64 >> wu) - 1);
+    }
     const int tile_pu = 1 << (wu + bu), tile_pv = (64 >> wu) * (4 >> bu);
-    t.u = tile_u * tile_pu + ((wave & ((1 << bu) - 1)) << wu) + (lane & ((1 << wu) - 1));
-    t.v = tile_v * tile_pv + (wave >> bu) * (64 >> wu) + (lane >> wu);
+    t.u = tile_u * tile_pu + ((wave & ((1 << bu) - 1)) << wu) + lu;
+    t.v = tile_v * tile_pv + (wave >> bu) * (64 >> wu) + lv;
     t.active = (t.u < P.nu) && (t.v < P.nv);
     return t;
 }
@@ -1383,10 +1440,8 @@ __device__ __forceinline__ void march_global(const MarchArgs &P, const RaySetup 
     for (int ka = R.k_lo & ~(kAnchor - 1); ka < k_hi; ka += kAnchor, fix_add(q, d16)) {
         const Anchor A = anchor_from(q, R);
         const int i1 = min(ka + kAnchor, k_hi) - ka;
-        int i = max(ka, R.k_lo) - ka;
-        for (float fi = (float)i; i < i1; i++, fi += 1.0f)
-            accumulate_global<M, ST, W>(rsrc, (const char *)P.vol, absolute_cell(A, offset_cell(A, fi), nx, ny, nz),
-                                        oy, oz, acc);
+        const int i = max(ka, R.k_lo) - ka;
+        gather_segment<M, ST, W, gather_samples(M, ST, 48)>(rsrc, (const char *)P.vol, A, i, i1, nx, ny, nz, oy, oz, acc);
     }
 }
 
@@ -1458,30 +1513,23 @@ __device__ __forceinline__ int row_max(int v)
     return max(v, __builtin_amdgcn_mov_dpp(v, 0x140, 0xF, 0xF, true));
 }
 
-// Ints of the march's box scratch: three buffers of 8 (lo x, y, z at 0..2,
-// hi x, y, z at 4..6).
-constexpr int kBoxBufs = 3;
-
-// Every box buffer back to (INT_MAX, INT_MIN); thread 0 only.
+// Ints of the march's block scratch: lo at 0..3, hi at 4..7.
 __device__ __forceinline__ void box_reset(int *buf)
 {
 #pragma unroll
-    for (int d = 0; d < 3; d++) {
+    for (int d = 0; d < 4; d++) {
         buf[d] = INT_MAX;
         buf[4 + d] = INT_MIN;
     }
 }
 
-// Block-wide min of lo[] and max of hi[] with one barrier, as scalars.  Each
-// 16-lane row reduces its lanes with DPP, one lane per row folds the row
-// into buffer `call` with LDS atomic min / max, and after the barrier every
-// lane reads it.  The buffer must be reset before the call; the call then
-// resets buffer call - 1 (mod 3), whose last reads all came before this
-// barrier, for use two calls later.
+// Block-wide min of lo[] and max of hi[], as scalars.  Each 16-lane row
+// reduces its lanes with DPP, one lane per row folds the row into `buf` with
+// LDS atomic min / max, and after the barrier every lane reads it.  The
+// buffer must be reset before the call.
 template <int D>
-__device__ __forceinline__ void block_box_atomic(int (&lo)[D], int (&hi)[D], int *boxbuf, int call)
+__device__ __forceinline__ void block_box_atomic(int (&lo)[D], int (&hi)[D], int *buf)
 {
-    int *buf = boxbuf + call * 8;
 #pragma unroll
     for (int d = 0; d < D; d++) {
         lo[d] = row_min(lo[d]);
@@ -1500,8 +1548,15 @@ __device__ __forceinline__ void block_box_atomic(int (&lo)[D], int (&hi)[D], int
         lo[d] = __builtin_amdgcn_readfirstlane(buf[d]);
         hi[d] = __builtin_amdgcn_readfirstlane(buf[4 + d]);
     }
-    if (threadIdx.x == 0) box_reset(boxbuf + (call == 0 ? kBoxBufs - 1 : call - 1) * 8);
 }
+
+// A float's place in the order of the floats as an int, and back (finite).
+__device__ __forceinline__ int float_key(float f)
+{
+    const int i = __float_as_int(f);
+    return i ^ ((i >> 31) & 0x7FFFFFFF);
+}
+__device__ __forceinline__ float key_float(int k) { return __int_as_float(k ^ ((k >> 31) & 0x7FFFFFFF)); }
 
 // Exact q = n / d for 0 <= n < 2^22, 1 <= d < 2^10, from a float reciprocal.
 __device__ __forceinline__ int small_div(int n, int d, float inv_d)
@@ -1515,8 +1570,40 @@ __device__ __forceinline__ int small_div(int n, int d, float inv_d)
 // 1 / d to within an ulp (v_rcp_f32); small_div corrects the quotient.
 __device__ __forceinline__ float small_rcp(int d) { return __builtin_amdgcn_rcpf((float)d); }
 
-// Rows a thread loads at once in fill_box.
-constexpr int kFillBatch = 4;
+// Row pitch and plane pitch (cells) of staged boxes of up to 14 x 15 cells a
+// plane: the y + 1 rows and z + 1 planes of a sample are then immediate LDS
+// offsets away.  Larger boxes (kDyn) use their own extents.
+constexpr int kRowPitch = 14;
+constexpr int kPlanePitch = 211; // 3 mod 16, see box_plane
+
+// Plane pitch (cells) of a staged box of sy rows of `pitch` cells: the next
+// value that is 3 mod 16.  The lanes of one
+// LDS pass read ~8 successive z planes at two (x, y) places (tile_lane); with
+// 3 (or 13) mod 16 their cells fall on different banks almost everywhere
+// (1.1 passes a read, against 2 to 2.6 with planes of 12 * sy cells).
+__device__ __forceinline__ int box_plane(int pitch, int sy) { return ((pitch * sy + 12) & ~15) + 3; }
+
+// One chunk of the march and the box staged for it (all block-uniform).
+struct Chunk {
+    int k0, n;            // samples [k0, k0 + n)
+    int lo[3];            // first cell
+    int sx, sy, sz;       // cells
+    int pitch, plane;     // in cells
+    bool staged, fixed;   // in LDS; at kRowPitch and kPlanePitch
+};
+
+// Of the next chunk's box, a wavefront keeps four quads of rows of this many
+// planes in flight while it marches the chunk before: 4 M registers a plane,
+// as many as fit beside the march (a spill waits for every load before it).
+// FP32 cells of three channels: one plane (3 x 512^3, 12 views: 8.6 ms; two
+// planes of three quads 9.3, none 8.8).
+constexpr int prefetch_planes(int M, int st, bool dyn)
+{
+    return dyn ? (M == 1 ? 3 : M == 2 ? 2 : 1) : M <= 2 ? 3 : st == kStF32 ? 1 : M == 3 ? 3 : 2;
+}
+// Planes whose loads a wavefront has in flight together, the kept ones
+// included (12 planes of the workgroup: most boxes whole).
+constexpr int kFillPlanes = 3;
 
 // An empty asm that reads one batch row's loaded dwords, placed after every
 // load of the batch is issued: the compiler waits for the batch there, once,
@@ -1535,121 +1622,179 @@ template <int M> __device__ __forceinline__ void loads_landed(const uint32_t (&c
         asm volatile("" ::"v"(c[0]), "v"(c[1]), "v"(c[2]), "v"(c[3]));
 }
 
-// Cooperative, row-coalesced load of the cell box [lo, lo + (sx, sy, sz)) into
-// LDS (cell (lx, row) of the box at byte (row * px + lx) * LB, x fastest;
-// row pitch px >= sx).  Cells outside the padded volume are zeros.  A thread
-// keeps one x column and walks rows (y, z) with a fixed stride, so the x test
-// and offset are hoisted and the loop holds no division.
-template <int M, bool W>
-__device__ __forceinline__ void fill_box(__amdgpu_buffer_rsrc_t rsrc, const char *vol, char *lds,
-                                         const int (&lo)[3], int sx, int px, int sy, int sz, int nx, int ny,
-                                         int nz, uint32_t oy, uint32_t oz)
-{
-    constexpr uint32_t LB = lds_cell_bytes<M>();
-    const int rows = sy * sz;
-    // A volume of 4 GiB or more (W): the buffer starts at plane zb, the box's
-    // first plane inside the padded volume, so every row offset stays
-    // 32-bit; offset 0 is still a padding (zero) cell.
-    uint32_t zb = 0;
-    if constexpr (W) {
-        const int pzn = nz + kVoxPadLo + kVoxPadHi;
-        zb = (uint32_t)min(max(lo[2] + kVoxPadLo, 0), pzn - 1);
-        const uint64_t rest = (uint64_t)(pzn - (int)zb) * oz;
-        rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(vol) + (uint64_t)zb * oz, 0,
-                                                 (int)(rest < 0xFFFFFFFFull ? rest : 0xFFFFFFFFull), 0x00020000);
+// The load of a chunk's cell box into LDS: cell (lx, ly, lz) of the box at
+// (lz * plane + ly * pitch + lx) * LB.  One load instruction of a wavefront
+// covers a quad of rows (y) of one plane, 16 cells of each: a lane's offset
+// within the quad is fixed for the whole box and the quad's own offset is a
+// scalar, so a quad costs a wavefront one load, one LDS write and two vector
+// adds.  (One thread per cell of a row-major walk took ~150 vector
+// instructions a chunk; buffer loads straight into LDS, which the three-dword
+// cell limits to one dword a lane, needed four times the load instructions.)
+// A wavefront takes every fourth plane.  Quad j of a plane is rows
+// min(4 j, sy - 4) .. + 3: the last may repeat rows, with the same values.
+// Cells outside the padded volume become zeros: their lanes read the padding
+// at offset 0.
+template <int M, bool W, int NZ> struct BoxFill {
+    static constexpr uint32_t LB = lds_cell_bytes<M>();
+    static constexpr int NW = kBlock / 64;
+    __amdgpu_buffer_rsrc_t rsrc;
+    uint32_t oy, oz;
+    int pxn, pyn, pzn, zb, X, Y, Z, quads, pitch, plane, sx, sy, sz, wave, lx, lr;
+    bool inside;
+
+    __device__ __forceinline__ BoxFill(const MarchArgs &P, __amdgpu_buffer_rsrc_t r, const Chunk &c)
+    {
+        rsrc = r;
+        oy = P.row_y & 0xFFFFFFu;
+        oz = P.row_z & 0xFFFFFFu;
+        pxn = P.pcx;
+        pyn = P.pcy;
+        pzn = P.pcz;
+        X = c.lo[0] + kVoxPadLo;
+        Y = c.lo[1] + kVoxPadLo;
+        Z = c.lo[2] + kVoxPadLo;
+        zb = 0;
+        if constexpr (W) {
+            // A volume of 4 GiB or more: the buffer starts at plane zb, the
+            // box's first plane inside the padded volume, so every row offset
+            // stays 32-bit; offset 0 is still a padding (zero) cell.
+            zb = min(max(Z, 0), pzn - 1);
+            const uint64_t rest = (uint64_t)(pzn - zb) * oz;
+            rsrc = __builtin_amdgcn_make_buffer_rsrc((char *)const_cast<void *>(P.vol) + (uint64_t)zb * oz, 0,
+                                                     (int)(rest < 0xFFFFFFFFull ? rest : 0xFFFFFFFFull), 0x00020000);
+        }
+        sx = c.sx;
+        sy = c.sy;
+        sz = c.sz;
+        pitch = c.pitch;
+        plane = c.plane;
+        quads = (sy + 3) >> 2;
+        inside = X >= 0 && X + sx <= pxn && Y >= 0 && Y + sy <= pyn && Z >= 0 && Z + sz <= pzn;
+        wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+        lx = threadIdx.x & 15;
+        lr = (threadIdx.x >> 4) & 3;
     }
-    if (sx <= kBlock) {
+
+    __device__ __forceinline__ bool large() const { return sx > 16 || sy > 16; }
+    __device__ __forceinline__ void store(char *lds, int lz, int y, const uint32_t (&d)[M]) const
+    {
+        lds_write<M>(lds, (uint32_t)(lr * pitch + lx) * LB + (uint32_t)(lz * plane + y * pitch) * LB, d);
+    }
+    // The first four quads of this wavefront's planes B .. B + N - 1 of a box
+    // inside the volume (a plane past the box repeats its last one; a uniform
+    // branch leaves out fourth quads).
+    template <int B, int N> __device__ __forceinline__ void load_planes(uint32_t (&d)[N][4][M]) const
+    {
+        const uint32_t voff = (uint32_t)(X + lx) * (4u * M) + __umul24((uint32_t)lr, oy);
+        uint32_t zo[N];
+#pragma unroll
+        for (int b = 0; b < N; b++) zo[b] = (uint32_t)(Z + min(wave + (B + b) * NW, sz - 1) - zb) * oz;
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            const uint32_t yo = (uint32_t)(Y + min(4 * j, sy - 4)) * oy;
+#pragma unroll
+            for (int b = 0; b < N; b++) load_raw<M>(rsrc, voff, zo[b] + yo, d[b][j]);
+        }
+        if (quads > 3) {
+            const uint32_t yo = (uint32_t)(Y + min(12, sy - 4)) * oy;
+#pragma unroll
+            for (int b = 0; b < N; b++) load_raw<M>(rsrc, voff, zo[b] + yo, d[b][3]);
+        }
+    }
+    template <int B, int N> __device__ __forceinline__ void store_planes(char *lds, const uint32_t (&d)[N][4][M]) const
+    {
+        if (lx < sx) {
+#pragma unroll
+            for (int b = 0; b < N; b++) {
+                const int lz = min(wave + (B + b) * NW, sz - 1);
+#pragma unroll
+                for (int j = 0; j < 3; j++) store(lds, lz, min(4 * j, sy - 4), d[b][j]);
+                if (quads > 3) store(lds, lz, min(12, sy - 4), d[b][3]);
+            }
+        }
+    }
+    // The box (of at most 16 cells and rows) of a chunk whose first NZ planes
+    // are in d (or in flight to it).
+    __device__ __forceinline__ void finish(char *lds, const uint32_t (&d)[NZ][4][M]) const
+    {
+        if (inside) { // block-uniform
+            constexpr int NR = kFillPlanes - NZ;
+            if constexpr (NR > 0) {
+                uint32_t r[NR][4][M];
+                load_planes<NZ, NR>(r);
+                store_planes<0, NZ>(lds, d);
+                store_planes<NZ, NR>(lds, r);
+            } else {
+                store_planes<0, NZ>(lds, d);
+            }
+        }
+        // boxes that reach out of the volume, and what is past those planes
+        const int x = X + lx;
+        for (int lz = inside ? wave + kFillPlanes * NW : wave; lz < sz; lz += NW) {
+            uint32_t r[4][M];
+            const int z = Z + lz;
+#pragma unroll
+            for (int b = 0; b < 4; b++) {
+                const int y = Y + min(4 * b, sy - 4) + lr;
+                const bool in = (uint32_t)x < (uint32_t)pxn && (uint32_t)y < (uint32_t)pyn && (uint32_t)z < (uint32_t)pzn;
+                load_raw<M>(rsrc, in ? __umul24((uint32_t)(z - zb), oz) + (__umul24((uint32_t)y, oy) + (uint32_t)x * (4u * M)) : 0u,
+                            0, r[b]);
+            }
+#pragma unroll
+            for (int b = 0; b < 4; b++) loads_landed<M>(r[b]);
+            if (lx < sx) {
+#pragma unroll
+                for (int b = 0; b < 4; b++) store(lds, lz, min(4 * b, sy - 4), r[b]);
+            }
+        }
+    }
+    // A box of more than 16 cells or rows (at most kBlock cells a row): a
+    // thread keeps one x column and walks the rows (y, z) with a fixed
+    // stride, so no lane is left over at a row's end and few round trips are
+    // made (192^3 FP32, one material, rays 1.1 voxels apart: 2.70 ms, 3.20 by
+    // row quads).
+    __device__ __forceinline__ void walk(char *lds) const
+    {
+        constexpr int NB = M == 1 ? 8 : 4;
         const float inv_sx = small_rcp(sx), inv_sy = small_rcp(sy);
         // rows per pass and its (y, z) step: block-uniform
         const int per = __builtin_amdgcn_readfirstlane(small_div(kBlock, sx, inv_sx));
         const int dz = __builtin_amdgcn_readfirstlane(small_div(per, sy, inv_sy)), dy = per - dz * sy;
         const int tid = threadIdx.x;
         if (tid >= per * sx) return;
-        const int r0 = small_div(tid, sx, inv_sx);
-        const int lx = tid - __mul24(r0, sx);
-        const int x = lo[0] + lx;
-        int lz = small_div(r0, sy, inv_sy);
-        int ly = r0 - __mul24(lz, sy);
-        const bool xin = (uint32_t)(x + kVoxPadLo) < (uint32_t)(nx + kVoxPadLo + kVoxPadHi);
-        const uint32_t xoff = ((uint32_t)(x + kVoxPadLo) & 0xFFFFFu) * (4u * M);
-        const uint32_t ymax = (uint32_t)(ny + kVoxPadLo + kVoxPadHi), zmax = (uint32_t)(nz + kVoxPadLo + kVoxPadHi);
-        uint32_t loff = (uint32_t)(__mul24(r0, px) + lx) * LB;
-        const uint32_t lstep = (uint32_t)(per * px) * LB;
-        // kFillBatch rows per pass of the loop: their loads are all in flight
-        // before the first LDS write.  A row outside the padded volume (or
-        // past the box) loads the padded cell at offset 0, which is a zero.
-        const bool inside = lo[0] >= -kVoxPadLo && lo[0] + sx <= nx + kVoxPadHi && lo[1] >= -kVoxPadLo &&
-                            lo[1] + sy <= ny + kVoxPadHi && lo[2] >= -kVoxPadLo && lo[2] + sz <= nz + kVoxPadHi;
-        if (inside) { // block-uniform: no row needs a bounds test
-            uint32_t off = __umul24((uint32_t)(lo[2] + lz + kVoxPadLo) - zb, oz) +
-                           (__umul24((uint32_t)(lo[1] + ly + kVoxPadLo), oy) + xoff);
-            const uint32_t step = (uint32_t)dy * oy + (uint32_t)dz * oz, wrap = oz - (uint32_t)sy * oy;
-            for (int r = r0; r < rows; r += kFillBatch * per) {
-                uint32_t d[kFillBatch][M];
+        const int rows = sy * sz, r0 = small_div(tid, sx, inv_sx), x = tid - __mul24(r0, sx);
+        int lz = small_div(r0, sy, inv_sy), ly = r0 - __mul24(lz, sy);
+        const bool xin = (uint32_t)(X + x) < (uint32_t)pxn;
+        const uint32_t xoff = ((uint32_t)(X + x) & 0xFFFFFu) * (4u * M);
+        uint32_t loff = (uint32_t)(__mul24(lz, plane) + __mul24(ly, pitch) + x) * LB;
+        const uint32_t lstep = (uint32_t)(dz * plane + dy * pitch) * LB, lwrap = (uint32_t)(plane - sy * pitch) * LB;
+        for (int r = r0; r < rows; r += NB * per) {
+            uint32_t d[NB][M], lo[NB];
 #pragma unroll
-                for (int b = 0; b < kFillBatch; b++) {
-                    load_raw<M>(rsrc, r + b * per < rows ? off : 0u, 0, d[b]);
-                    ly += dy;
-                    off += step;
-                    if (ly >= sy) {
-                        ly -= sy;
-                        off += wrap;
-                    }
-                }
-#pragma unroll
-                for (int b = 0; b < kFillBatch; b++) loads_landed<M>(d[b]);
-#pragma unroll
-                for (int b = 0; b < kFillBatch; b++) {
-                    if (r + b * per < rows) lds_write<M>(lds, loff, d[b]);
-                    loff += lstep;
-                }
-            }
-            return;
-        }
-        for (int r = r0; r < rows; r += kFillBatch * per) {
-            uint32_t d[kFillBatch][M];
-#pragma unroll
-            for (int b = 0; b < kFillBatch; b++) {
-                const uint32_t yi = (uint32_t)(lo[1] + ly + kVoxPadLo), zi = (uint32_t)(lo[2] + lz + kVoxPadLo);
-                const bool in = xin && yi < ymax && zi < zmax;
-                load_raw<M>(rsrc, in ? __umul24(zi - zb, oz) + (__umul24(yi, oy) + xoff) : 0u, 0, d[b]);
+            for (int b = 0; b < NB; b++) {
+                // a row outside the padded volume (or past the box) loads the
+                // padded cell at offset 0, which is a zero
+                const uint32_t yi = (uint32_t)(Y + ly), zi = (uint32_t)(Z + lz);
+                const bool in = xin && yi < (uint32_t)pyn && zi < (uint32_t)pzn && r + b * per < rows;
+                load_raw<M>(rsrc, in ? __umul24(zi - (uint32_t)zb, oz) + (__umul24(yi, oy) + xoff) : 0u, 0, d[b]);
+                lo[b] = loff;
                 ly += dy;
                 lz += dz;
+                loff += lstep;
                 if (ly >= sy) {
                     ly -= sy;
                     lz++;
+                    loff += lwrap;
                 }
             }
 #pragma unroll
-            for (int b = 0; b < kFillBatch; b++) loads_landed<M>(d[b]);
+            for (int b = 0; b < NB; b++) loads_landed<M>(d[b]);
 #pragma unroll
-            for (int b = 0; b < kFillBatch; b++) {
-                if (r + b * per < rows) lds_write<M>(lds, loff, d[b]);
-                loff += lstep;
-            }
-        }
-    } else {
-        const int cells = rows * sx;
-        const float inv_sx = small_rcp(sx), inv_sy = small_rcp(sy);
-        for (int i = threadIdx.x; i < cells; i += kBlock) {
-            const int row = small_div(i, sx, inv_sx), lx = i - row * sx;
-            const int lz = small_div(row, sy, inv_sy), ly = row - lz * sy;
-            const int x = lo[0] + lx, y = lo[1] + ly, z = lo[2] + lz;
-            uint32_t d[M];
-            if (x >= -kVoxPadLo && x < nx + kVoxPadHi && y >= -kVoxPadLo && y < ny + kVoxPadHi &&
-                z >= -kVoxPadLo && z < nz + kVoxPadHi) {
-                const uint32_t xi = (uint32_t)(x + kVoxPadLo) & 0xFFFFFu;
-                const uint32_t yi = (uint32_t)(y + kVoxPadLo) & 0xFFFFFu;
-                const uint32_t zi = (uint32_t)(z + kVoxPadLo) & 0xFFFFFu;
-                load_raw<M>(rsrc, (zi - zb) * oz + (yi * oy + xi * (4u * M)), 0, d);
-            } else {
-#pragma unroll
-                for (int m = 0; m < M; m++) d[m] = 0u;
-            }
-            lds_write<M>(lds, (uint32_t)(row * px + lx) * LB, d);
+            for (int b = 0; b < NB; b++)
+                if (r + b * per < rows) lds_write<M>(lds, lo[b], d[b]);
         }
     }
-}
+};
 
 // a * b + c for |a|, |b| < 2^23 (v_mad_i32_i24, one full-rate instruction;
 // written out because the compiler otherwise emits two multiplies and a
@@ -1661,53 +1806,108 @@ __device__ __forceinline__ int mad_i24(int a, int b, int c)
     return r;
 }
 
-// The samples of one chunk from its staged box (row pitch PX cells, or px
-// when PX is 0; plane pitch pitch * sy).  A sample's cell offset from the
-// anchor's cell becomes one cell index and then bytes; the y + 1 rows lie
-// one row pitch further (an immediate offset when PX is fixed) and the
-// z + 1 rows one plane further.
-template <int M, int ST, int PX>
-__device__ __forceinline__ void march_staged(const RaySetup &R, const Anchor &A0, FixPos q, const FixPos &d16,
-                                             int k0, int chunk, int c_lo, int c_hi, const int (&lo)[3], int px,
-                                             int sy, const char *lds, float (&acc)[M])
+// The samples of one chunk from its staged box (row pitch PX cells and plane
+// pitch PZ cells, or `pitch` and `plane` where they are 0).  A sample's cell
+// offset from the anchor's cell becomes one byte offset; the y + 1 rows lie
+// one row pitch and the z + 1 rows one plane further (immediate LDS offsets
+// where the pitches are fixed).  q is the position of the anchor at or before
+// k0, and becomes that of the anchor at or before k1.
+//
+// The planes of sample s + 1 are read as those of sample s are used, so the
+// LDS round trip (~100 cycles) runs under the ~40 instructions of a sample.
+// An empty asm takes every dword of a plane's cells where they are first
+// needed: without it the pad dword of a three-channel cell counts as dead at
+// once, the compiler puts a temporary into its register, and that write has
+// to wait for the read (two exposed round trips a sample: a third of the
+// march's wave cycles).
+template <int M, int ST, int PX, int PZ>
+__device__ __forceinline__ void march_staged(const RaySetup &R, FixPos &q, const FixPos &d16, int k0, int k1,
+                                             int c_lo, int c_hi, const int (&lo)[3], int pitch, int plane,
+                                             const char *lds, float (&acc)[M])
 {
-    constexpr uint32_t LB = lds_cell_bytes<M>();
-    const int pitch = PX > 0 ? PX : px;
-    const int plane = pitch * sy;
-    const uint32_t ry = (uint32_t)pitch * LB, rz = (uint32_t)plane * LB;
-    for (int ka = k0; ka < k0 + chunk; ka += kAnchor, fix_add(q, d16)) {
+    constexpr int LB = (int)lds_cell_bytes<M>();
+    constexpr int NP = kPlaneCells<ST>;
+    typedef typename CellWords<M>::type words;
+    typedef const __attribute__((address_space(3))) words lds_words;
+    struct Plane {
+        words w[NP];
+    };
+    if constexpr (PX > 0) pitch = PX;
+    if constexpr (PZ > 0) plane = PZ;
+    const int ry = pitch * LB, rz = plane * LB;
+    const int base = (int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char *)lds -
+                     (lo[2] * rz + lo[1] * ry + lo[0] * LB);
+    for (int ka = k0 & ~(kAnchor - 1); ka < k1; ka += kAnchor) {
         const int i1 = min(ka + kAnchor, c_hi) - ka;
         int i = max(ka, c_lo) - ka;
+        const Anchor A = anchor_from(q, R);
+        if (ka + kAnchor <= k1) fix_add(q, d16); // block-uniform
         if (i >= i1) continue;
-        const Anchor A = ka == k0 ? A0 : anchor_from(q, R);
-        // the anchor's cell in the box
-        const char *pa = lds + (((A.ic - lo[2]) * sy + (A.ib - lo[1])) * pitch + (A.ia - lo[0])) * (int)LB;
-        auto sample = [&](float fi) {
-            const Cell c = offset_cell(A, fi);
-            const int ci = mad_i24(c.z, plane, mad_i24(c.y, pitch, c.x));
-            const char *p0 = pa + ci * (int)LB;
-            const char *p2 = p0 + rz;
-            accumulate<M, ST>(c, [&](int r, uint32_t(&out)[M]) {
-                lds_read<M>((r & 2) ? p2 : p0, ((r & 1) ? ry : 0u) + (r < 4 ? 0u : LB), out);
+        // LDS address of the anchor's cell
+        const int pa = base + (A.ic * rz + A.ib * ry + A.ia * LB);
+        auto locate = [&](float fi, Cell &c) {
+            c = offset_cell(A, fi);
+            return mad_i24(c.z, rz, mad_i24(c.y, ry, pa + c.x * LB));
+        };
+        auto read = [&](int p, Plane &k) {
+#pragma unroll
+            for (int r = 0; r < NP; r++)
+                k.w[r] = *(lds_words *)(uintptr_t)(uint32_t)(p + (ST == kStF32 ? (r >> 1) * ry + (r & 1) * LB : r * ry));
+        };
+        auto add = [&](Plane &k, const Cell &c, int z) {
+            if constexpr (M == 3) {
+#pragma unroll
+                for (int r = 0; r < NP; r++) asm("" : "+v"(k.w[r]));
+            }
+            add_plane<M, ST>(c, z, [&](int r, int m) {
+                if constexpr (M == 1)
+                    return k.w[r];
+                else
+                    return k.w[r][m];
             }, acc);
         };
         if (i == 0 && i1 == kAnchor) { // a whole segment (most of them)
+            Cell c[2];
+            int p = locate(0.0f, c[0]);
+            Plane z0, z1;
+            read(p, z0);
+            read(p + rz, z1);
 #pragma unroll
-            for (int s = 0; s < kAnchor; s++) sample((float)s);
+            for (int s = 0; s < kAnchor; s++) {
+                const bool more = s + 1 < kAnchor;
+                if (more) p = locate((float)(s + 1), c[(s + 1) & 1]);
+                add(z0, c[s & 1], 0);
+                if (more) read(p, z0);
+                add(z1, c[s & 1], 1);
+                if (more) read(p + rz, z1);
+                // keeps the order: hoisted across samples, the reads and
+                // positions of many samples would not fit the registers
+                __builtin_amdgcn_sched_barrier(0);
+            }
         } else {
-            for (float fi = (float)i; i < i1; i++, fi += 1.0f) sample(fi);
+            float fi = (float)i;
+            for (; i < i1; i++, fi += 1.0f) {
+                Cell c;
+                const int p = locate(fi, c);
+                Plane z0, z1;
+                read(p, z0);
+                read(p + rz, z1);
+                add(z0, c, 0);
+                add(z1, c, 1);
+            }
         }
     }
 }
 
-// True when every cell the chunk's box [lo, hi] stages (16-bit cells hold
-// the x + 1 voxel, so one cell fewer in x) is zero in every channel: all
-// bricks of the occupancy grid that overlap the box, clipped to the padded
-// volume, are empty (cells outside it read the padding's zeros).  The chunk
-// would add exact zeros to every ray, so it can be skipped.  Every wave
-// computes the same answer from the block-uniform box, one brick per lane.
+// True when every cell of the box [lo, hi] (16-bit cells hold the x + 1
+// voxel, so one cell fewer in x) is zero in every channel: all bricks of the
+// occupancy grid that overlap the box, clipped to the padded volume, are
+// empty (cells outside it read the padding's zeros).  A chunk with such a
+// box would add exact zeros to every ray, so it can be skipped.  A lane's own
+// box: four bricks of a row per (unaligned) load.
+constexpr int kEmptyBricks = 4; // a box of more bricks on an axis is marched
 template <int ST>
-__device__ __forceinline__ bool chunk_empty(const MarchArgs &P, const int (&lo)[3], const int (&hi)[3])
+__device__ __forceinline__ bool box_empty(const MarchArgs &P, const int (&lo)[3], const int (&hi)[3])
 {
     const int x0 = max(lo[0] + kVoxPadLo, 0), x1 = min(hi[0] + kVoxPadLo - (ST == kStF32 ? 0 : 1), P.pcx - 1);
     const int y0 = max(lo[1] + kVoxPadLo, 0), y1 = min(hi[1] + kVoxPadLo, P.pcy - 1);
@@ -1715,108 +1915,218 @@ __device__ __forceinline__ bool chunk_empty(const MarchArgs &P, const int (&lo)[
     if (x0 > x1 || y0 > y1 || z0 > z1) return true;
     const int bx0 = x0 / kOccBrick, by0 = y0 / kOccBrick, bz0 = z0 / kOccBrick;
     const int nbx = x1 / kOccBrick - bx0 + 1, nby = y1 / kOccBrick - by0 + 1, nbz = z1 / kOccBrick - bz0 + 1;
-    if (nbx > 4 || nby > 4 || nbz > 4) return false; // a box this large is marched
-    const int lane = threadIdx.x & 63;
-    const int jx = lane & 3, jy = (lane >> 2) & 3, jz = lane >> 4;
-    bool any = false;
-    // 24-bit products: a padded volume has fewer than 2^24 bricks per axis
-    // and fewer than 2^32 in all (2^41 cells)
-    if (jx < nbx && jy < nby && jz < nbz)
-        any = P.occ[__umul24(__umul24((uint32_t)(bz0 + jz), (uint32_t)P.ob_y) + (uint32_t)(by0 + jy),
-                             (uint32_t)P.ob_x) +
-                    (uint32_t)(bx0 + jx)] != 0;
-    return __builtin_amdgcn_ballot_w64(any) == 0;
+    if (nbx > kEmptyBricks || nby > kEmptyBricks || nbz > kEmptyBricks) return false;
+    uint32_t any = 0;
+#pragma unroll
+    for (int jz = 0; jz < kEmptyBricks; jz++)
+#pragma unroll
+        for (int jy = 0; jy < kEmptyBricks; jy++) {
+            // (rows past the box repeat its last one)
+            const uint32_t r = __umul24((uint32_t)(bz0 + min(jz, nbz - 1)), (uint32_t)P.ob_y) + (uint32_t)(by0 + min(jy, nby - 1));
+            uint32_t four;
+            __builtin_memcpy(&four, P.occ + ((uint64_t)r * (uint32_t)P.ob_x + (uint32_t)bx0), 4);
+            any |= four;
+        }
+    return (any & (0xFFFFFFFFu >> (8 * (kEmptyBricks - nbx)))) == 0;
 }
 
 // Ray-march of one block's rays with the volume staged in LDS per chunk of
 // samples: the rays move together along the common sample lattice; for each
-// chunk of `chunk` samples the box of cells they touch is loaded once,
-// row-coalesced, and all 8 (or 4) corner reads come from LDS.  A chunk whose
-// box exceeds the LDS budget reads from global memory instead.  Each ray still
-// accumulates in ascending k, so the result equals march_kernel's bit for bit.
-// Every thread of the block must call it (it synchronises the block).
+// chunk the box of cells they can touch is loaded once, row by row, and all 8
+// (or 4) corner reads come from LDS.  A chunk holds P.chunk samples, or fewer
+// where the box of that many would not fit the LDS budget (down to 4: pixels
+// or steps of many voxels); a box that still does not fit reads from global
+// memory instead.  Each ray accumulates in ascending k whatever the
+// chunks, so the result equals march_kernel's bit for bit.  Every thread of
+// the block must call it (it synchronises the block).
+// kDyn: boxes may be of any extents; without it a chunk whose box is not
+// within kRowPitch x (kPlanePitch / kRowPitch) cells a plane is split.
 // kCount: no fill and no march; `marched` receives the lane's samples in the
 // chunks that would be marched (the decisions are the march's own).
-template <int M, int ST, bool W, bool kCount = false>
-__device__ __forceinline__ void march_chunks(const MarchArgs &P, const RaySetup &R,
+template <int M, int ST, bool W, bool kDyn, bool kCount = false>
+__device__ __forceinline__ void march_chunks(const MarchArgs &P, const TileLane &t, const RaySetup &R,
                                              __amdgpu_buffer_rsrc_t rsrc, char *lds, int *boxbuf,
                                              float (&acc)[M], int *marched = nullptr)
 {
     const uint32_t oy = P.row_y & 0xFFFFFFu, oz = P.row_z & 0xFFFFFFu;
     const int nx = (int)P.nx, ny = (int)P.ny, nz = (int)P.nz;
     const int k_hi = R.k_lo + R.n;
-    int kr_lo[1] = {R.n > 0 ? R.k_lo : INT_MAX}, kr_hi[1] = {R.n > 0 ? k_hi : INT_MIN};
-    // the block's previous users of the scratch have finished two barriers
-    // ago; the barrier below publishes the reset buffers
-    if (threadIdx.x == 0) {
+    // the block's sample range and its range of steps on each axis
+    int blo[4], bhi[4];
+    blo[0] = R.n > 0 ? R.k_lo : INT_MAX;
+    bhi[0] = R.n > 0 ? k_hi : INT_MIN;
 #pragma unroll
-        for (int b = 0; b < kBoxBufs; b++) box_reset(boxbuf + 8 * b);
+    for (int a = 0; a < 3; a++) {
+        const int key = float_key(R.df[a]);
+        blo[1 + a] = R.n > 0 ? key : INT_MAX;
+        bhi[1 + a] = R.n > 0 ? key : INT_MIN;
+    }
+    __syncthreads(); // the block's previous users of the scratch are done
+    if (threadIdx.x == 0) box_reset(boxbuf);
+    __syncthreads();
+    block_box_atomic<4>(blo, bhi, boxbuf);
+    const int kb_hi = bhi[0];
+    if (blo[0] >= kb_hi) return; // no ray of the block has samples (block-uniform)
+    const int kstart = blo[0] & ~(kAnchor - 1);
+    // The cell box of the tile's rays as it moves along the sample lattice.
+    // Every ray of the tile starts at the view's source S, so at sample k its
+    // position on an axis is S + (tau + k) D with tau = t0 / dx > 0 and D its
+    // step, and the tile's positions lie between S + (tau + k) Dmin and
+    // S + (tau + k) Dmax: two lines an axis, evaluated for each chunk, in
+    // place of a reduction over the block's rays and a barrier per chunk.
+    // Lanes 0..2 compute the lower lines, 3..5 the upper ones, as FP32 from
+    // sample kstart on; they wait in the scratch (registers are dear).
+    const int lane = threadIdx.x & 63;
+    float *lines = (float *)(boxbuf + 8); // [6]: at kstart, per sample, 1 where it moves outwards, 0
+    if (threadIdx.x < 6) {
+        double S[3];
+        ray_source(P, (int)(P.view_begin + t.vw_local), S[0], S[1], S[2]);
+        const int ax = lane % 3;
+        const bool up = lane >= 3;
+        const double src = ax == 0 ? S[0] : ax == 1 ? S[1] : S[2];
+        const float d = key_float(up ? (ax == 0 ? bhi[1] : ax == 1 ? bhi[2] : bhi[3]) : (ax == 0 ? blo[1] : ax == 1 ? blo[2] : blo[3]));
+        const double sign = up ? 1.0 : -1.0, D = (double)d, k = P.t0 / P.dx + (double)kstart;
+        // widened by the steps' rounding to FP32 (2^-24 relative) over the
+        // way from the source, by that of the lines' own FP32 arithmetic over
+        // the volume, and by the march's positions (~1e-6 max(1, step) voxel)
+        const double margin = 1e-3 + 6e-7 * (double)(P.nx + P.ny + P.nz) + fabs(D) * (4e-6 + 6.1e-8 * k);
+        lines[4 * lane] = (float)(src + D * k + sign * margin);
+        lines[4 * lane + 1] = d;
+        lines[4 * lane + 2] = (up ? d > 0.0f : d < 0.0f) ? 1.0f : 0.0f;
     }
     __syncthreads();
-    int call = 0;
-    block_box_atomic<1>(kr_lo, kr_hi, boxbuf, call);
-    const int kb_hi = kr_hi[0];
-    // the chunk's first anchor walks in exact fixed-point steps
-    const int kstart = kr_lo[0] & ~(kAnchor - 1);
-    const FixPos d16 = fix_steps(R, kAnchor), dchunk = fix_steps(R, P.chunk);
+    // a line's bound (a cell) over samples [k0, k0 + n), kk = k0 - kstart
+    auto bound = [&](int l, float kk, int n) {
+        const float *q = lines + 4 * l;
+        return floor_to_int(fmaf(q[1], fmaf(q[2], (float)(n - 1), kk), q[0]));
+    };
+    // the anchor at or before the chunk walks in exact fixed-point steps
+    const FixPos d16 = fix_steps(R, kAnchor);
     FixPos pk = fix_at(R, kstart);
-    // chunks start on the anchor grid (chunk is a multiple of kAnchor)
-    for (int k0 = kstart; k0 < kb_hi; k0 += P.chunk, fix_add(pk, dchunk)) {
-        const int c_lo = max(k0, R.k_lo), c_hi = min(k0 + P.chunk, k_hi);
-        // the chunk's cell box from the lane's FP32 sample positions; the
-        // first anchor is kept for the march
-        int lo[3] = {INT_MAX, INT_MAX, INT_MAX}, hi[3] = {INT_MIN, INT_MIN, INT_MIN};
-        const Anchor A0 = anchor_from(pk, R);
-        {
-            const int i0 = max(k0, c_lo) - k0, i1 = min(k0 + kAnchor, c_hi) - k0;
-            if (i0 < i1) segment_box(A0, i0, i1, lo, hi);
-        }
-        {
-            FixPos q = pk;
-            for (int ka = k0 + kAnchor; ka < k0 + P.chunk; ka += kAnchor) {
-                fix_add(q, d16);
-                const int i0 = max(ka, c_lo) - ka, i1 = min(ka + kAnchor, c_hi) - ka;
-                if (i0 < i1) segment_box(anchor_from(q, R), i0, i1, lo, hi);
+    int ka = kstart; // the anchor pk stands at
+    const int cells = P.lds_cells;
+    // bit i: the i-th next chunk of P.chunk samples holds only zero cells; 64
+    // chunks at a time, one lane each
+    uint64_t skip = 0;
+    int left = 0; // chunks of `skip` not yet used
+    int unit = kstart; // where the next P.chunk samples start
+    bool gather = false; // a box was far too large (they grow along the rays)
+    // the first chunk from k0 on that is not empty (k0 >= kb_hi: none)
+    auto next_chunk = [&](int k0) {
+        Chunk c;
+        if (k0 == unit) {
+            for (; P.occ && k0 < kb_hi; k0 += P.chunk) {
+                if (left == 0) {
+                    // the boxes of the next 64 chunks, one per lane
+                    const float kk = (float)(k0 - kstart + lane * P.chunk);
+                    int lo[3], hi[3];
+#pragma unroll
+                    for (int a = 0; a < 3; a++) {
+                        lo[a] = bound(a, kk, P.chunk);
+                        hi[a] = bound(3 + a, kk, P.chunk) + 1;
+                    }
+                    bool empty = false;
+                    if (k0 + (int64_t)lane * P.chunk < kb_hi) empty = box_empty<ST>(P, lo, hi);
+                    skip = __builtin_amdgcn_ballot_w64(empty);
+                    left = 64;
+                }
+                const bool empty = skip & 1;
+                skip >>= 1;
+                left--;
+                if (!empty) break;
             }
+            unit = k0 + P.chunk;
         }
-        // every wave has finished the previous chunk past this barrier
-        call = call == kBoxBufs - 1 ? 0 : call + 1;
-        block_box_atomic<3>(lo, hi, boxbuf, call);
-        if (hi[0] < lo[0]) continue; // no lane of the block samples this chunk (block-uniform)
-        if (P.occ && chunk_empty<ST>(P, lo, hi)) continue; // all zeros (block-uniform)
-        if constexpr (kCount) {
-            *marched += max(0, c_hi - c_lo);
-            continue;
+        c.k0 = k0;
+        // up to the unit's end, or a part of an anchor's segment
+        const int off = k0 & (kAnchor - 1);
+        c.n = off ? off & -off : unit - k0;
+        c.staged = false;
+        if (k0 >= kb_hi || gather) return c;
+        for (;;) {
+            const int v = bound(lane < 6 ? lane : 5, (float)(k0 - kstart), c.n);
+            int hi[3];
+#pragma unroll
+            for (int a = 0; a < 3; a++) {
+                c.lo[a] = __builtin_amdgcn_readlane(v, a);
+                hi[a] = __builtin_amdgcn_readlane(v, 3 + a) + 1; // the +1 corner
+            }
+            // 16-bit cells are x-pairs that already hold the +1 x corner
+            c.sx = hi[0] - c.lo[0] + (ST == kStF32 ? 1 : 0);
+            c.sy = max(4, hi[1] - c.lo[1] + 1); // rows are filled four at a time
+            c.sz = hi[2] - c.lo[2] + 1;
+            c.pitch = kDyn ? max(c.sx, kRowPitch) : kRowPitch;
+            // (a box of a volume past 4 GiB is staged only if its planes span
+            // less than 4 GiB, so its row offsets fit 32 bits)
+            c.fixed = c.sx <= kRowPitch && c.sy * kRowPitch <= kPlanePitch && c.sz <= cells && kPlanePitch * c.sz <= cells;
+            c.staged = c.fixed;
+            if constexpr (kDyn)
+                c.staged |= c.sx <= kBlock && c.sy <= cells && c.sz <= cells && box_plane(c.pitch, c.sy) <= cells &&
+                            box_plane(c.pitch, c.sy) * c.sz <= cells;
+            if constexpr (W) c.staged &= (uint64_t)c.sz * oz < 0xFFFFFFFFull;
+            if (c.staged) break;
+            if (c.n <= 4) {
+                c.n = off ? off & -off : unit - k0;
+                gather = c.sy > cells || c.sz > cells || c.sx * c.sy > cells ||
+                         c.sx * c.sy * c.sz > cells + cells / 4;
+                break;
+            }
+            c.n = c.n > kAnchor ? max(kAnchor, (c.n / 2) & ~(kAnchor - 1)) : c.n / 2;
         }
-        // 16-bit cells are x-pairs that already hold the +1 x corner
-        const int sx = hi[0] - lo[0] + (ST == kStF32 ? 1 : 0), sy = hi[1] - lo[1] + 1, sz = hi[2] - lo[2] + 1;
-        // (a box of a volume past 4 GiB is staged only if its planes span
-        // less than 4 GiB, so its row offsets fit 32 bits)
-        const bool staged = (int64_t)sx * sy * sz <= (int64_t)P.lds_cells &&
-                            (!W || (uint64_t)sz * oz < 0xFFFFFFFFull);
-        if (staged) {
-            // Row pitch: 12 cells for boxes up to 12 wide when that still
-            // fits (then the y + 1 rows are an immediate LDS offset away),
-            // sx otherwise (block-uniform).
-            const int px = sx <= 12 && (int64_t)12 * sy * sz <= (int64_t)P.lds_cells ? 12 : sx;
-            fill_box<M, W>(rsrc, (const char *)P.vol, lds, lo, sx, px, sy, sz, nx, ny, nz, oy, oz);
-            __syncthreads();
-            if (px == 12)
-                march_staged<M, ST, 12>(R, A0, pk, d16, k0, P.chunk, c_lo, c_hi, lo, px, sy, lds, acc);
+        c.plane = c.fixed || !kDyn ? kPlanePitch : box_plane(c.pitch, c.sy);
+        return c;
+    };
+    if constexpr (kCount) {
+        for (int k0 = kstart;;) {
+            const Chunk c = next_chunk(k0);
+            if (c.k0 >= kb_hi) return;
+            k0 = c.k0 + c.n;
+            *marched += max(0, min(k0, k_hi) - max(c.k0, R.k_lo));
+        }
+    }
+    // the next chunk's box is on its way while a chunk is marched
+    constexpr int NZ = prefetch_planes(M, ST, kDyn);
+    uint32_t d[NZ][4][M];
+    Chunk c = next_chunk(kstart);
+    auto prefetch = [&](const Chunk &q) {
+        const BoxFill<M, W, NZ> f(P, rsrc, q);
+        if (q.staged && f.inside && !(kDyn && f.large())) f.template load_planes<0, NZ>(d);
+    };
+    prefetch(c);
+    while (c.k0 < kb_hi) {
+        if (c.staged) {
+            __syncthreads(); // every wave has finished with the box before
+            const BoxFill<M, W, NZ> f(P, rsrc, c);
+            if (kDyn && f.large())
+                f.walk(lds);
             else
-                march_staged<M, ST, 0>(R, A0, pk, d16, k0, P.chunk, c_lo, c_hi, lo, px, sy, lds, acc);
+                f.finish(lds, d);
+            __syncthreads();
+        }
+        const Chunk next = next_chunk(c.k0 + c.n);
+        prefetch(next);
+        for (; ka + kAnchor <= c.k0; ka += kAnchor) fix_add(pk, d16); // past empty chunks
+        const int k1 = c.k0 + c.n;
+        const int c_lo = max(c.k0, R.k_lo), c_hi = min(k1, k_hi);
+        if (c.staged) {
+            if (!kDyn || c.fixed)
+                march_staged<M, ST, kRowPitch, kPlanePitch>(R, pk, d16, c.k0, k1, c_lo, c_hi, c.lo, c.pitch, c.plane, lds, acc);
+            else if constexpr (kDyn)
+                march_staged<M, ST, 0, 0>(R, pk, d16, c.k0, k1, c_lo, c_hi, c.lo, c.pitch, c.plane, lds, acc);
         } else {
             FixPos q = pk;
-            for (int ka = k0; ka < k0 + P.chunk; ka += kAnchor, fix_add(q, d16)) {
-                const int i1 = min(ka + kAnchor, c_hi) - ka;
-                int i = max(ka, c_lo) - ka;
-                if (i >= i1) continue;
-                const Anchor A = ka == k0 ? A0 : anchor_from(q, R);
-                for (float fi = (float)i; i < i1; i++, fi += 1.0f)
-                    accumulate_global<M, ST, W>(rsrc, (const char *)P.vol,
-                                                absolute_cell(A, offset_cell(A, fi), nx, ny, nz), oy, oz, acc);
+            for (int kq = ka; kq < k1; kq += kAnchor) {
+                const int i1 = min(kq + kAnchor, c_hi) - kq;
+                const int i = max(kq, c_lo) - kq;
+                const Anchor A = anchor_from(q, R);
+                if (kq + kAnchor <= k1) fix_add(q, d16);
+                gather_segment<M, ST, W, kDyn ? gather_samples(M, ST, 32) : 1>(rsrc, (const char *)P.vol, A, i, i1, nx, ny, nz, oy,
+                                                                          oz, acc);
             }
+            pk = q;
         }
+        ka = k1 & ~(kAnchor - 1);
+        c = next;
     }
 }
 
@@ -1829,32 +2139,41 @@ __device__ __forceinline__ RaySetup lane_ray(const MarchArgs &P, const TileLane 
 
 // One ray tile (logical block `logical` of P) through the LDS-staged march.
 // The first 256 bytes of `lds_raw` are block scratch, the rest staged cells.
-// kWide: also instantiate the march for volumes of 4 GiB or more (the batch
-// kernel, which inlines every material count, leaves it out).
-template <int M, int ST, bool kSpectrum, bool kWide = true>
+// kDyn, kWide: boxes of any extents, volumes of 4 GiB or more (the code for
+// them costs registers, so launches that need neither leave it out).
+template <int M, int ST, bool kSpectrum, bool kDyn, bool kWide>
 __device__ __forceinline__ void march_tile(const MarchArgs &P, uint32_t logical, char *lds_raw)
 {
-    const TileLane t = tile_lane(P, logical);
-    const RaySetup R = lane_ray<true>(P, t);
-    __amdgpu_buffer_rsrc_t rsrc =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(P.vol), 0, (int)P.vol_bytes, 0x00020000);
     float acc[M];
 #pragma unroll
     for (int m = 0; m < M; m++) acc[m] = 0.0f;
-    if (kWide && P.wide)
-        march_chunks<M, ST, kWide>(P, R, rsrc, lds_raw + 256, (int *)lds_raw, acc);
-    else
-        march_chunks<M, ST, false>(P, R, rsrc, lds_raw + 256, (int *)lds_raw, acc);
-    finish_ray<M, ST, kSpectrum>(P, t, acc);
+    {
+        const TileLane t = tile_lane(P, logical);
+        const RaySetup R = lane_ray<true>(P, t);
+        __amdgpu_buffer_rsrc_t rsrc =
+            __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(P.vol), 0, (int)P.vol_bytes, 0x00020000);
+        if (kWide && P.wide)
+            march_chunks<M, ST, kWide, kDyn>(P, t, R, rsrc, lds_raw + 256, (int *)lds_raw, acc);
+        else
+            march_chunks<M, ST, false, kDyn>(P, t, R, rsrc, lds_raw + 256, (int *)lds_raw, acc);
+    }
+    // the lane's pixel again, not kept in registers through the march
+    asm("" : "+s"(logical));
+    finish_ray<M, ST, kSpectrum>(P, tile_lane(P, logical), acc);
 }
 
-template <int M, int ST, bool kSpectrum>
+// The march's kernels by what a launch needs (box_kind): boxes of at most
+// 14 x 15 cells a plane; boxes of any extents; those and volumes of 4 GiB or
+// more.
+enum BoxKind { kBoxFixed = 0, kBoxDyn = 1, kBoxWide = 2 };
+
+template <int M, int ST, bool kSpectrum, int kKind>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void march_lds_kernel(MarchArgs P)
 {
     extern __shared__ char lds_raw[];
     const uint32_t logical = xcd_logical(P);
     if (logical >= P.n_blocks) return;
-    march_tile<M, ST, kSpectrum>(P, logical, lds_raw);
+    march_tile<M, ST, kSpectrum, kKind != kBoxFixed, kKind == kBoxWide>(P, logical, lds_raw);
 }
 
 // Samples the march evaluates (each ray's clipped window [k_lo, k_hi)),
@@ -1893,7 +2212,7 @@ __global__ __launch_bounds__(kBlock) void count_marched_kernel(MarchArgs P, unsi
         __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(P.vol), 0, (int)P.vol_bytes, 0x00020000);
     float acc[1] = {0.0f};
     int marched = 0;
-    march_chunks<1, ST, false, true>(P, R, rsrc, nullptr, boxbuf, acc, &marched);
+    march_chunks<1, ST, false, true, true>(P, t, R, rsrc, nullptr, boxbuf, acc, &marched);
     unsigned long long n = (unsigned long long)marched;
 #pragma unroll
     for (int s = 32; s >= 1; s >>= 1) n += __shfl_xor(n, s);
@@ -1919,7 +2238,6 @@ constexpr int kXcds = 8;
 
 struct BatchItem {
     MarchArgs P;
-    int32_t n_mat;
 };
 
 struct BatchQueues {
@@ -1933,11 +2251,11 @@ __global__ void batch_reset(uint32_t *taken, int n)
     for (int i = threadIdx.x; i < n; i += blockDim.x) taken[i] = 0u;
 }
 
-template <int ST>
+template <int M, int ST, bool kDyn>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void batch_kernel(const BatchItem *__restrict__ items, BatchQueues Q)
 {
     extern __shared__ char lds_raw[];
-    uint32_t *slot = (uint32_t *)lds_raw + 60; // beside the march's box scratch (ints 0..23)
+    uint32_t *slot = (uint32_t *)lds_raw + 60; // beside the march's box scratch (ints 0..31)
     const uint32_t home = blockIdx.x & (kXcds - 1);
     const int stride = Q.n_items + 1;
     for (uint32_t qi = 0; qi < (uint32_t)kXcds; qi++) {
@@ -1956,12 +2274,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
             const uint32_t r = u - base[i];
             const uint32_t tiles = (uint32_t)(it.P.tiles_u * it.P.tiles_v);
             const uint32_t logical = ((r / tiles) * kXcds + x) * tiles + r % tiles;
-            switch (it.n_mat) {
-            case 1: march_tile<1, ST, true, false>(it.P, logical, lds_raw); break;
-            case 2: march_tile<2, ST, true, false>(it.P, logical, lds_raw); break;
-            case 3: march_tile<3, ST, true, false>(it.P, logical, lds_raw); break;
-            default: march_tile<4, ST, true, false>(it.P, logical, lds_raw); break;
-            }
+            march_tile<M, ST, true, kDyn, false>(it.P, logical, lds_raw);
         }
     }
 }
@@ -1972,7 +2285,7 @@ using BatchFn = void (*)(const BatchItem *, BatchQueues);
 
 struct AdjointArgs {
     const float *gI, *gIA; // [views][nv][nu] or null (zero)
-    const float *L;        // [views][M][nv][nu] or null (recomputed)
+    const float *L;        // [views][M][nv][nu]
     float *grad;           // [M][nz][ny][nx], accumulated
 };
 
@@ -2086,36 +2399,19 @@ __device__ __forceinline__ void scatter_chunks(const MarchArgs &P, const RaySetu
     }
 }
 
-// Adjoint of ctfp_forward for upstream gradients gI, gIA: per ray, the line
-// integrals (read or recomputed), then dl/dL_m = (gIA - gI) sum_e A[e][m]
-// W_e e^-tau_e, then the backprojection of dx * dl/dL_m.
-// dl/dL_m * dx of the lane's ray: the line integrals (read from G.L or
-// recomputed by the march), then (gIA - gI) sum_e A[e][m] W_e e^-tau_e dx.
-// Every thread of the block must call it (the march synchronises).
-template <int M, int ST>
-__device__ __forceinline__ void ray_gradient(const MarchArgs &P, const AdjointArgs &G, const TileLane &t,
-                                             const RaySetup &R, char *lds_raw, float (&g)[M])
+// Adjoint of ctfp_forward for upstream gradients gI, gIA: per ray, from its
+// line integrals, dl/dL_m = (gIA - gI) sum_e A[e][m] W_e e^-tau_e, then the
+// backprojection of dx * dl/dL_m.
+// dl/dL_m * dx of the lane's ray.
+template <int M>
+__device__ __forceinline__ void ray_gradient(const MarchArgs &P, const AdjointArgs &G, const TileLane &t, float (&g)[M])
 {
     const int64_t npix = (int64_t)P.nu * P.nv;
     const int64_t pix = (int64_t)t.v * P.nu + t.u;
     float Lm[M];
-    if (G.L) {
 #pragma unroll
-        for (int m = 0; m < M; m++)
-            Lm[m] = t.active ? G.L[((int64_t)t.vw_local * M + m) * npix + pix] : 0.0f;
-    } else {
-        __amdgpu_buffer_rsrc_t rsrc =
-            __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(P.vol), 0, (int)P.vol_bytes, 0x00020000);
-        float acc[M];
-#pragma unroll
-        for (int m = 0; m < M; m++) acc[m] = 0.0f;
-        if (P.wide)
-            march_chunks<M, ST, true>(P, R, rsrc, lds_raw + 256, (int *)lds_raw, acc);
-        else
-            march_chunks<M, ST, false>(P, R, rsrc, lds_raw + 256, (int *)lds_raw, acc);
-#pragma unroll
-        for (int m = 0; m < M; m++) Lm[m] = acc[m] * P.dx_f;
-    }
+    for (int m = 0; m < M; m++)
+        Lm[m] = t.active ? G.L[((int64_t)t.vw_local * M + m) * npix + pix] : 0.0f;
 #pragma unroll
     for (int m = 0; m < M; m++) g[m] = 0.0f;
     if (t.active) {
@@ -2157,18 +2453,16 @@ __device__ __forceinline__ void ray_gradient(const MarchArgs &P, const AdjointAr
 }
 
 // Ray pass of the gather adjoint: writes dl/dL_m * dx per ray into
-// gL [view - view_begin][m][v][u].
-template <int M, int ST>
+// gL [view - view_begin][m][v][u] (which may be G.L itself: a thread reads
+// its ray's line integrals before it writes).
+template <int M>
 __global__ __launch_bounds__(kBlock) void ray_grad_kernel(MarchArgs P, AdjointArgs G, float *gL)
 {
-    extern __shared__ char lds_raw[];
     const uint32_t logical = xcd_logical(P);
     if (logical >= P.n_blocks) return;
     const TileLane t = tile_lane(P, logical);
-    // the ray's samples only when its line integrals are recomputed
-    const RaySetup R = G.L ? empty_ray() : lane_ray<true>(P, t);
     float g[M];
-    ray_gradient<M, ST>(P, G, t, R, lds_raw, g);
+    ray_gradient<M>(P, G, t, g);
     if (t.active) {
         const int64_t npix = (int64_t)P.nu * P.nv;
         const int64_t pix = (int64_t)t.v * P.nu + t.u;
@@ -2788,7 +3082,7 @@ __global__ __launch_bounds__(256) void cell_combine_kernel(const float *__restri
     }
 }
 
-template <int M, int ST>
+template <int M>
 __global__ __launch_bounds__(kBlock) void adjoint_kernel(MarchArgs P, AdjointArgs G)
 {
     extern __shared__ char lds_raw[];
@@ -2797,7 +3091,7 @@ __global__ __launch_bounds__(kBlock) void adjoint_kernel(MarchArgs P, AdjointArg
     const TileLane t = tile_lane(P, logical);
     const RaySetup R = lane_ray(P, t);
     float g[M];
-    ray_gradient<M, ST>(P, G, t, R, lds_raw, g);
+    ray_gradient<M>(P, G, t, g);
     scatter_chunks<M>(P, R, g, G.grad, lds_raw + 256, (int *)lds_raw);
 }
 
@@ -2864,12 +3158,16 @@ __global__ __launch_bounds__(kBlock) void ray_grad_from_l_kernel(MarchArgs P, Ad
 
 using MarchFn = void (*)(MarchArgs);
 
-template <int ST> MarchFn pick_march_st(int n_mat, bool spectrum, bool lds)
+template <int ST> MarchFn pick_march_st(int n_mat, bool spectrum, bool lds, int kind)
 {
-#define CTFP_PICK(Mv)                                                                   \
-    case Mv:                                                                            \
-        if (lds) return spectrum ? march_lds_kernel<Mv, ST, true> : march_lds_kernel<Mv, ST, false>; \
-        return spectrum ? march_kernel<Mv, ST, true> : march_kernel<Mv, ST, false>;
+#define CTFP_PICK_KIND(Mv, Kv) \
+    return spectrum ? march_lds_kernel<Mv, ST, true, Kv> : march_lds_kernel<Mv, ST, false, Kv>
+#define CTFP_PICK(Mv)                                                                          \
+    case Mv:                                                                                   \
+        if (!lds) return spectrum ? march_kernel<Mv, ST, true> : march_kernel<Mv, ST, false>;  \
+        if (kind == kBoxFixed) CTFP_PICK_KIND(Mv, kBoxFixed);                                  \
+        if (kind == kBoxDyn) CTFP_PICK_KIND(Mv, kBoxDyn);                                      \
+        CTFP_PICK_KIND(Mv, kBoxWide);
     switch (n_mat) {
         CTFP_PICK(1)
         CTFP_PICK(2)
@@ -2878,29 +3176,20 @@ template <int ST> MarchFn pick_march_st(int n_mat, bool spectrum, bool lds)
     default: return nullptr;
     }
 #undef CTFP_PICK
+#undef CTFP_PICK_KIND
 }
 
 using AdjointFn = void (*)(MarchArgs, AdjointArgs);
 using RayGradFn = void (*)(MarchArgs, AdjointArgs, float *);
 using GatherFn = void (*)(GatherArgs);
 
-template <int ST> RayGradFn pick_ray_grad_st(int n_mat)
+RayGradFn pick_ray_grad(int n_mat)
 {
     switch (n_mat) {
-    case 1: return ray_grad_kernel<1, ST>;
-    case 2: return ray_grad_kernel<2, ST>;
-    case 3: return ray_grad_kernel<3, ST>;
-    case 4: return ray_grad_kernel<4, ST>;
-    default: return nullptr;
-    }
-}
-
-RayGradFn pick_ray_grad(int n_mat, int dtype)
-{
-    switch (dtype) {
-    case CTFP_F32: return pick_ray_grad_st<kStF32>(n_mat);
-    case CTFP_F16: return pick_ray_grad_st<kStF16>(n_mat);
-    case CTFP_BF16: return pick_ray_grad_st<kStBF16>(n_mat);
+    case 1: return ray_grad_kernel<1>;
+    case 2: return ray_grad_kernel<2>;
+    case 3: return ray_grad_kernel<3>;
+    case 4: return ray_grad_kernel<4>;
     default: return nullptr;
     }
 }
@@ -2939,33 +3228,23 @@ CombineFn pick_cell_combine(int n_mat)
     }
 }
 
-template <int ST> AdjointFn pick_adjoint_st(int n_mat)
+AdjointFn pick_adjoint(int n_mat)
 {
     switch (n_mat) {
-    case 1: return adjoint_kernel<1, ST>;
-    case 2: return adjoint_kernel<2, ST>;
-    case 3: return adjoint_kernel<3, ST>;
-    case 4: return adjoint_kernel<4, ST>;
+    case 1: return adjoint_kernel<1>;
+    case 2: return adjoint_kernel<2>;
+    case 3: return adjoint_kernel<3>;
+    case 4: return adjoint_kernel<4>;
     default: return nullptr;
     }
 }
 
-AdjointFn pick_adjoint(int n_mat, int dtype)
+MarchFn pick_march(int n_mat, int dtype, bool spectrum, bool lds, int kind)
 {
     switch (dtype) {
-    case CTFP_F32: return pick_adjoint_st<kStF32>(n_mat);
-    case CTFP_F16: return pick_adjoint_st<kStF16>(n_mat);
-    case CTFP_BF16: return pick_adjoint_st<kStBF16>(n_mat);
-    default: return nullptr;
-    }
-}
-
-MarchFn pick_march(int n_mat, int dtype, bool spectrum, bool lds)
-{
-    switch (dtype) {
-    case CTFP_F32: return pick_march_st<kStF32>(n_mat, spectrum, lds);
-    case CTFP_F16: return pick_march_st<kStF16>(n_mat, spectrum, lds);
-    case CTFP_BF16: return pick_march_st<kStBF16>(n_mat, spectrum, lds);
+    case CTFP_F32: return pick_march_st<kStF32>(n_mat, spectrum, lds, kind);
+    case CTFP_F16: return pick_march_st<kStF16>(n_mat, spectrum, lds, kind);
+    case CTFP_BF16: return pick_march_st<kStBF16>(n_mat, spectrum, lds, kind);
     default: return nullptr;
     }
 }
@@ -3048,7 +3327,8 @@ static int alloc_volume_buffers(ctfp_context *ctx, size_t bytes, int64_t obx, in
         dfree(ctx->obox);
         dfree(ctx->odist);
     }
-    if (!ctx->occ) HIP_TRY(dev_malloc(&ctx->occ, (size_t)(obx * oby * obz) * n_groups));
+    // (the march reads rows of bricks four at a time)
+    if (!ctx->occ) HIP_TRY(dev_malloc(&ctx->occ, (size_t)(obx * oby * obz) * n_groups + 4));
     if (!ctx->obox) HIP_TRY(dev_malloc(&ctx->obox, (size_t)n_groups * 6 * sizeof(int32_t)));
     if (!ctx->odist) HIP_TRY(dev_malloc(&ctx->odist, (size_t)(obx * oby * obz) * (n_groups + 1)));
     return CTFP_OK;
@@ -3713,6 +3993,71 @@ static int spectral_args(ctfp_context *ctx, MarchArgs &P)
     return CTFP_OK;
 }
 
+// What the march of a channel group needs: its kernel and its LDS.
+struct BoxPlan {
+    int kind;     // BoxKind
+    int lds;      // bytes per workgroup
+    bool gathers; // most chunks are too large to stage
+};
+
+// Bytes of a channel group's cell in LDS.
+static int lds_cell(int mats) { return mats == 3 ? 16 : 4 * mats; }
+
+// The kernel and the LDS follow from how far apart a tile's rays are in
+// voxels.
+//  - A volume of 4 GiB or more has its own kernel.
+//  - When no box of 8 samples exceeds kRowPitch x (kPlanePitch / kRowPitch)
+//    cells a plane, the fixed-box kernel runs (it splits a chunk whose box
+//    does): three of a sample's 44 instructions and ~20 registers less than
+//    with boxes of any extents.  The bound: the tile's pixels at the far side
+//    of the volume and 8 samples along them, at the worst angle in the plane,
+//    and along z.  Its LDS is what such boxes of 16 samples need, at most the
+//    budget; one-channel cells are 4 bytes, and more workgroups share a CU.
+//  - Otherwise the budget grows to the first of 52 and 64 KiB (3 and 2
+//    workgroups a CU) that holds a typical box of 8 samples (the middle of the
+//    volume, rays at 45 degrees, and a tenth more), where a smaller one would
+//    leave most chunks to the global gather; past 1.15 times 64 KiB most are
+//    gathered anyway, with the budget that was asked for (more wavefronts; a
+//    kernel without boxes and with more loads in flight was 7 % slower on
+//    3 x 160^3 FP32 at 1.14 voxel, 40 % with yet more wavefronts: the gather
+//    is bound by what its rays share in the caches): 3 x 192^3 FP32, pixels 0.73 voxel apart, 60 views,
+//    5.2 ms with 40 KiB, 3.6 with 52, 4.7 with 64; 3 x 160^3 FP16, 0.85
+//    voxel, 40 views, 1.95, 1.27 and 1.24 ms.
+static BoxPlan box_plan(const ctfp_context *ctx, int group)
+{
+    const ctfp_scan_params &s = ctx->scan;
+    const ctfp_system_info &y = ctx->sys;
+    const int cell = lds_cell(ctx->group_mats[group]), budget = ctx->tune.lds_bytes;
+    const int xc = ctx->dtype == CTFP_F32 ? 3 : 2; // 16-bit cells hold the +1 x corner
+    // (pixels spread with the depth along the central ray)
+    const double hx = y.p_half_x + y.p_size_x, hy = y.p_half_y + y.p_size_y;
+    const double far = ((double)s.sod + std::sqrt(hx * hx + hy * hy)) * 1.002;
+    const double nu = (double)ctx->tune.wave_u * ctx->tune.block_u - 1;
+    const double nv = 64.0 / ctx->tune.wave_u * (4.0 / ctx->tune.block_u) - 1;
+    const double slope = (double)y.d_half_lv / s.sdd; // of a ray towards z
+    // floor(a + length) - floor(a) + 2 cells of a length, at most
+    auto count = [](double length, int more) { return (int)std::min(1e6, std::floor(length + 0.02)) + more; };
+    const double pix = (double)s.d_size * far / s.sdd, mid = (double)s.d_size * s.sod / s.sdd;
+    const double d8 = 7.0 * y.dx, d16 = 15.0 * y.dx;
+    const bool wide = ctx->group_bytes[group] >= 0xFFFFFFFFull;
+    const double plane = std::sqrt(nu * pix * nu * pix + d8 * d8);
+    const int need_z = count((nv * pix + d16 * slope) / y.p_size_z, 3);
+    const int fits = (budget - 256) / cell;
+    if (!wide && count(plane / y.p_size_x, xc) <= kRowPitch && count(plane / y.p_size_y, 3) * kRowPitch <= kPlanePitch &&
+        (int64_t)count((nv * pix + d8 * slope) / y.p_size_z, 3) * kPlanePitch <= fits)
+        return {kBoxFixed, std::min(budget, 256 + need_z * kPlanePitch * cell), false};
+    const double side = (nu * mid + d8) * std::sqrt(0.5);
+    const int bx = std::max(kRowPitch, count(side / y.p_size_x, xc)), by = std::max(4, count(side / y.p_size_y, 3));
+    const int bz = count((nv * mid + d8 * slope) / y.p_size_z, 3);
+    const double need = 256.0 + cell * ((double)bx * by + 16.0) * bz;
+    int lds = budget;
+    if (lds < 1.1 * need) lds = std::max(lds, 52 * 1024);
+    if (lds < 1.1 * need) lds = std::max(lds, 64 * 1024);
+    // mostly gathered: no more LDS than asked for, so more wavefronts
+    const bool gathers = 1.15 * lds < need;
+    return {wide ? kBoxWide : kBoxDyn, gathers ? budget : lds, gathers};
+}
+
 // Launch arguments of the march of channel group `group` over views
 // [view_begin, view_begin + count): with the spectrum (I, IA; one group
 // only) and / or the line integrals into L [count][n_mat][v][u].
@@ -3731,10 +4076,12 @@ static int forward_args(ctfp_context *ctx, int64_t view_begin, int64_t view_coun
     P.I = I;
     P.IA = IA;
     P.L = L;
-    const int mg = ctx->group_mats[group];
-    const uint32_t lb = mg == 3 ? 16u : 4u * (uint32_t)mg;
     P.chunk = ctx->tune.chunk;
-    P.lds_cells = (int32_t)((ctx->tune.lds_bytes - 256) / lb);
+    const BoxPlan plan = box_plan(ctx, group);
+    P.lds_cells = (plan.lds - 256) / lds_cell(ctx->group_mats[group]);
+    // (1- and 2-channel cells in boxes of any extents: 2 to 3 % slower with it)
+    P.pass_order = ctx->tune.march == CTFP_MARCH_LDS && !plan.gathers &&
+                   (plan.kind == kBoxFixed || ctx->group_mats[group] > 2);
     return CTFP_OK;
 }
 
@@ -3745,9 +4092,10 @@ static int launch_group(ctfp_context *ctx, int64_t view_begin, int64_t view_coun
 {
     const bool lds = ctx->tune.march == CTFP_MARCH_LDS;
     if (!ctx->vol) return set_error(CTFP_ERR_STATE, "no volumes uploaded");
-    MarchFn fn = pick_march(ctx->group_mats[group], ctx->dtype, spectrum, lds);
+    const BoxPlan plan = box_plan(ctx, group);
+    MarchFn fn = pick_march(ctx->group_mats[group], ctx->dtype, spectrum, lds, plan.kind);
     if (!fn) return set_error(CTFP_ERR_UNSUPPORTED, "n_mat=%d", ctx->group_mats[group]);
-    const size_t shmem = lds ? (size_t)ctx->tune.lds_bytes : 0;
+    const size_t shmem = lds ? (size_t)plan.lds : 0;
     const int64_t npix = ctx->scan.d_num_u * ctx->scan.d_num_v;
     const int64_t per = views_per_launch(ctx);
     DeviceGuard g(ctx->device);
@@ -3908,8 +4256,8 @@ static int backward_impl(ctfp_context *ctx, int64_t view_begin, int64_t view_cou
     // which needs no buffer of corner sums
     const bool cell = ctx->tune.adjoint == CTFP_ADJOINT_CELL && !ws;
     const bool grouped = ctx->n_groups > 1;
-    // CTFP_MARCH_GLOBAL: no chunk is staged; every sample gathers and
-    // scatters through global memory (the LDS then only holds the box scratch)
+    // CTFP_MARCH_GLOBAL: the scatter stages no chunk; every sample scatters
+    // through global memory (the LDS then only holds the box scratch)
     const bool global = ctx->tune.march == CTFP_MARCH_GLOBAL;
     const size_t shmem = global ? 256 : (size_t)ctx->tune.lds_bytes;
     const ctfp_scan_params &s = ctx->scan;
@@ -3919,9 +4267,25 @@ static int backward_impl(ctfp_context *ctx, int64_t view_begin, int64_t view_cou
         if (grouped)
             return set_error(CTFP_ERR_UNSUPPORTED, "the scatter adjoint takes up to %d materials (%d given); use "
                              "the gather", kGroupMats, ctx->n_mat);
-        AdjointFn fn = pick_adjoint(ctx->n_mat, ctx->dtype);
+        AdjointFn fn = pick_adjoint(ctx->n_mat);
         if (!fn) return set_error(CTFP_ERR_UNSUPPORTED, "n_mat=%d", ctx->n_mat);
-        const int64_t per = views_per_launch(ctx);
+        int64_t per = views_per_launch(ctx);
+        float *lws = nullptr;
+        if (!L) {
+            // the line integrals of a group of views, marched first
+            const int64_t one = (int64_t)ctx->n_mat * npix * (int64_t)sizeof(float);
+            if (ws) {
+                per = std::min<int64_t>(per, (int64_t)ws_bytes / one);
+                if (per < 1)
+                    return set_error(CTFP_ERR_UNSUPPORTED, "line integrals of one view (%lld bytes) exceed the %lld-byte "
+                                     "static workspace", (long long)one, (long long)ws_bytes);
+                lws = ws;
+            } else {
+                per = std::max<int64_t>(1, std::min<int64_t>({per, view_count, (int64_t)kLWorkspaceBytes / one}));
+                if ((rc = ensure_l_ws(ctx, per))) return rc;
+                lws = ctx->l_ws;
+            }
+        }
         for (int64_t v0 = 0; v0 < view_count; v0 += per) {
             const int64_t n = std::min(per, view_count - v0);
             MarchArgs Q;
@@ -3930,8 +4294,9 @@ static int backward_impl(ctfp_context *ctx, int64_t view_begin, int64_t view_cou
             const uint32_t lb = ctx->n_mat == 3 ? 16u : 4u * (uint32_t)ctx->n_mat;
             Q.chunk = ctx->tune.chunk;
             Q.lds_cells = global ? 0 : (int32_t)((ctx->tune.lds_bytes - 256) / lb);
+            if (lws && (rc = launch_group(ctx, view_begin + v0, n, nullptr, nullptr, lws, stream, false, 0))) return rc;
             AdjointArgs G{gI ? gI + v0 * npix : nullptr, gIAbsorb ? gIAbsorb + v0 * npix : nullptr,
-                          L ? L + v0 * ctx->n_mat * npix : nullptr, grad};
+                          L ? L + v0 * ctx->n_mat * npix : lws, grad};
             hipLaunchKernelGGL(fn, dim3(Q.per_xcd * 8), dim3(kBlock), shmem, (hipStream_t)stream, Q, G);
             HIP_TRY(hipGetLastError());
         }
@@ -3939,7 +4304,7 @@ static int backward_impl(ctfp_context *ctx, int64_t view_begin, int64_t view_cou
     }
     // gather: per group of views, the ray pass writes dl/dL * dx into the
     // workspace and the voxel pass adds its backprojection to grad
-    RayGradFn rfn = grouped ? nullptr : pick_ray_grad(ctx->n_mat, ctx->dtype);
+    RayGradFn rfn = grouped ? nullptr : pick_ray_grad(ctx->n_mat);
     if (!grouped && !rfn) return set_error(CTFP_ERR_UNSUPPORTED, "n_mat=%d", ctx->n_mat);
     const int64_t per_view = (int64_t)ctx->n_mat * npix * (int64_t)sizeof(float);
     // more than four materials without L: the line integrals of the group
@@ -4005,10 +4370,13 @@ static int backward_impl(ctfp_context *ctx, int64_t view_begin, int64_t view_cou
             MarchArgs Q;
             if ((rc = fill_march_args(ctx, view_begin + v0, n, Q))) return rc;
             if ((rc = spectral_args(ctx, Q))) return rc;
-            const uint32_t lb = ctx->n_mat == 3 ? 16u : 4u * (uint32_t)ctx->n_mat;
-            Q.chunk = ctx->tune.chunk;
-            Q.lds_cells = global ? 0 : (int32_t)((ctx->tune.lds_bytes - 256) / lb);
-            hipLaunchKernelGGL(rfn, dim3(Q.per_xcd * 8), dim3(kBlock), shmem, (hipStream_t)stream, Q, G, ws);
+            if (!L) {
+                // marched into the workspace, which the ray pass then turns
+                // into dl/dL in place
+                if ((rc = launch_group(ctx, view_begin + v0, n, nullptr, nullptr, ws, stream, false, 0))) return rc;
+                G.L = ws;
+            }
+            hipLaunchKernelGGL(rfn, dim3(Q.per_xcd * 8), dim3(kBlock), 0, (hipStream_t)stream, Q, G, ws);
             HIP_TRY(hipGetLastError());
         } else {
             const float *Lc = G.L;
@@ -4312,13 +4680,17 @@ int ctfp_autotune(ctfp_context *ctx, int max_lds_bytes, ctfp_tuning *best)
 } // extern "C"
 
 struct ctfp_batch {
-    // items of one LDS budget share a persistent launch (and its occupancy)
+    // items of one material count, kernel and LDS (box_plan) share a
+    // persistent launch
     struct Group {
         BatchItem *d_items = nullptr;
         uint32_t *d_base = nullptr; // [kXcds][n + 1]
         int n = 0;
         size_t shmem = 0;
         unsigned grid = 0;
+        BatchFn fn = nullptr;
+        hipStream_t stream = nullptr; // of its branch while capturing
+        hipEvent_t done = nullptr;
     };
     int device = 0;
     int dtype = CTFP_F32;
@@ -4333,6 +4705,7 @@ struct ctfp_batch {
     float *l_ws = nullptr;
     size_t l_ws_bytes = 0;
     hipStream_t cap_stream = nullptr;
+    hipEvent_t fork = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     int64_t samples = 0;
@@ -4345,7 +4718,10 @@ void batch_free(ctfp_batch *b)
     if (b->exec) (void)hipGraphExecDestroy(b->exec);
     if (b->graph) (void)hipGraphDestroy(b->graph);
     if (b->cap_stream) (void)hipStreamDestroy(b->cap_stream);
+    if (b->fork) (void)hipEventDestroy(b->fork);
     for (auto &g : b->groups) {
+        if (g.stream) (void)hipStreamDestroy(g.stream);
+        if (g.done) (void)hipEventDestroy(g.done);
         dfree(g.d_items);
         dfree(g.d_base);
     }
@@ -4354,12 +4730,23 @@ void batch_free(ctfp_batch *b)
     delete b;
 }
 
-BatchFn pick_batch(int dtype)
+template <int ST> BatchFn pick_batch_st(int n_mat, bool dyn)
+{
+    switch (n_mat) {
+    case 1: return dyn ? batch_kernel<1, ST, true> : batch_kernel<1, ST, false>;
+    case 2: return dyn ? batch_kernel<2, ST, true> : batch_kernel<2, ST, false>;
+    case 3: return dyn ? batch_kernel<3, ST, true> : batch_kernel<3, ST, false>;
+    case 4: return dyn ? batch_kernel<4, ST, true> : batch_kernel<4, ST, false>;
+    default: return nullptr;
+    }
+}
+
+BatchFn pick_batch(int n_mat, int dtype, bool dyn)
 {
     switch (dtype) {
-    case CTFP_F32: return batch_kernel<kStF32>;
-    case CTFP_F16: return batch_kernel<kStF16>;
-    case CTFP_BF16: return batch_kernel<kStBF16>;
+    case CTFP_F32: return pick_batch_st<kStF32>(n_mat, dyn);
+    case CTFP_F16: return pick_batch_st<kStF16>(n_mat, dyn);
+    case CTFP_BF16: return pick_batch_st<kStBF16>(n_mat, dyn);
     default: return nullptr;
     }
 }
@@ -4409,21 +4796,42 @@ int ctfp_batch_create(const ctfp_batch_item *items, int n_items, ctfp_batch **ou
             int rc = forward_args(c, items[i].view_begin, items[i].view_count, items[i].I, items[i].IAbsorb,
                                   nullptr, true, h[i].P);
             if (rc) return rc;
-            h[i].n_mat = c->n_mat;
         }
         samples += items[i].view_count * c->scan.d_num_u * c->scan.d_num_v * c->sys.int_num;
     }
     auto is_grouped = [&](int i) { return std::find(grouped.begin(), grouped.end(), i) != grouped.end(); };
-    // groups by LDS budget, in order of first appearance
-    std::vector<int> budgets;
+    // groups by materials, kernel and LDS, in order of first appearance
+    struct Kind {
+        int n_mat, kind, lds;
+        bool operator==(const Kind &o) const { return n_mat == o.n_mat && kind == o.kind && lds == o.lds; }
+    };
+    std::vector<Kind> kinds;
+    // Side by side or one after the other.  A scan that gathers waits for
+    // memory where a staged one issues arithmetic, so the two share the CUs
+    // well, if their workgroups take equal LDS (a smaller one's leaves holes
+    // that the other's do not fit): a batch of five, two of them gathering,
+    // 14.3 ms one after the other, 9.7 side by side, 10.7 with unequal LDS.
+    // Launches of few tiles a workgroup hide each other's last tiles (two
+    // scans of 96^3, 16 tiles: 895 us, 850 side by side).  Larger staged scans
+    // only share the L2: 96^3, 192^3 and 128^3 FP32, 70 tiles, 4.81 ms and
+    // 5.24 side by side.
+    bool gathers = false;
+    int64_t tiles = 0;
     for (int i = 0; i < n_items; i++)
-        if (!is_grouped(i) &&
-            std::find(budgets.begin(), budgets.end(), items[i].ctx->tune.lds_bytes) == budgets.end())
-            budgets.push_back(items[i].ctx->tune.lds_bytes);
+        if (!is_grouped(i)) {
+            gathers |= box_plan(items[i].ctx, 0).gathers;
+            tiles += (int64_t)h[i].P.tiles_u * h[i].P.tiles_v * h[i].P.n_views;
+        }
+    auto kind_of = [&](int i) {
+        const BoxPlan p = box_plan(items[i].ctx, 0);
+        return Kind{items[i].ctx->n_mat, p.kind, gathers ? std::max(p.lds, items[i].ctx->tune.lds_bytes) : p.lds};
+    };
+    for (int i = 0; i < n_items; i++)
+        if (!is_grouped(i) && std::find(kinds.begin(), kinds.end(), kind_of(i)) == kinds.end()) kinds.push_back(kind_of(i));
     DeviceGuard g(c0->device);
-    BatchFn fn = pick_batch(c0->dtype);
     hipDeviceProp_t prop;
     HIP_TRY(hipGetDeviceProperties(&prop, c0->device));
+    const bool beside = kinds.size() > 1 && (gathers || tiles < 32 * 4 * (int64_t)prop.multiProcessorCount);
     ctfp_batch *b = new ctfp_batch();
     b->device = c0->device;
     b->dtype = c0->dtype;
@@ -4442,10 +4850,11 @@ int ctfp_batch_create(const ctfp_batch_item *items, int n_items, ctfp_batch **ou
         if (e != hipSuccess) return fail(hip_status(e), hipGetErrorString(e));
         b->l_ws_bytes = l_ws_bytes;
     }
-    for (int budget : budgets) {
+    for (const auto &kind : kinds) {
+        const int budget = kind.lds;
         std::vector<BatchItem> gi;
         for (int i = 0; i < n_items; i++)
-            if (!is_grouped(i) && items[i].ctx->tune.lds_bytes == budget) gi.push_back(h[i]);
+            if (!is_grouped(i) && kind_of(i) == kind) gi.push_back(h[i]);
         const int n = (int)gi.size();
         std::vector<uint32_t> base((size_t)kXcds * (n + 1), 0u);
         for (int i = 0; i < n; i++) {
@@ -4461,8 +4870,9 @@ int ctfp_batch_create(const ctfp_batch_item *items, int n_items, ctfp_batch **ou
         ctfp_batch::Group grp;
         grp.n = n;
         grp.shmem = (size_t)std::max(budget, 256);
+        grp.fn = pick_batch(kind.n_mat, c0->dtype, kind.kind != kBoxFixed);
         int per_cu = 0;
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kBlock, grp.shmem);
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, grp.fn, kBlock, grp.shmem);
         if (e != hipSuccess) return fail(CTFP_ERR_DEVICE, hipGetErrorString(e));
         if (per_cu < 1) return fail(CTFP_ERR_UNSUPPORTED, "kernel does not fit a CU");
         grp.grid = std::max(8u, (unsigned)(per_cu * prop.multiProcessorCount) / 8 * 8);
@@ -4481,6 +4891,11 @@ int ctfp_batch_create(const ctfp_batch_item *items, int n_items, ctfp_batch **ou
     // per group, then the items of more than four materials) is captured
     // once on a private stream and replayed
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->cap_stream, hipStreamNonBlocking);
+    if (e == hipSuccess && beside) e = hipEventCreateWithFlags(&b->fork, hipEventDisableTiming);
+    for (int k = 1; beside && k < ng && e == hipSuccess; k++) {
+        e = hipStreamCreateWithFlags(&b->groups[k].stream, hipStreamNonBlocking);
+        if (e == hipSuccess) e = hipEventCreateWithFlags(&b->groups[k].done, hipEventDisableTiming);
+    }
     if (e == hipSuccess) e = hipStreamBeginCapture(b->cap_stream, hipStreamCaptureModeThreadLocal);
     int grc = CTFP_OK;
     if (e == hipSuccess) {
@@ -4489,12 +4904,21 @@ int ctfp_batch_create(const ctfp_batch_item *items, int n_items, ctfp_batch **ou
             batch_reset<<<1, 256, 0, b->cap_stream>>>(b->d_taken, ng * kXcds);
             launch = hipGetLastError();
         }
+        // side by side: one branch of the graph per persistent kernel
+        if (beside && launch == hipSuccess) launch = hipEventRecord(b->fork, b->cap_stream);
         for (int k = 0; k < ng && launch == hipSuccess; k++) {
             const ctfp_batch::Group &grp = b->groups[k];
+            const bool branch = beside && k > 0;
+            const hipStream_t st = branch ? grp.stream : b->cap_stream;
             BatchQueues Q{b->d_taken + k * kXcds, grp.d_base, grp.n};
-            hipLaunchKernelGGL(fn, dim3(grp.grid), dim3(kBlock), grp.shmem, b->cap_stream, grp.d_items, Q);
+            if (branch) launch = hipStreamWaitEvent(st, b->fork, 0);
+            if (launch != hipSuccess) break;
+            hipLaunchKernelGGL(grp.fn, dim3(grp.grid), dim3(kBlock), grp.shmem, st, grp.d_items, Q);
             launch = hipGetLastError();
+            if (branch && launch == hipSuccess) launch = hipEventRecord(grp.done, st);
         }
+        for (int k = 1; beside && k < ng && launch == hipSuccess; k++)
+            launch = hipStreamWaitEvent(b->cap_stream, b->groups[k].done, 0);
         for (size_t k = 0; k < grouped.size() && launch == hipSuccess && grc == CTFP_OK; k++) {
             const ctfp_batch_item &it = items[grouped[k]];
             grc = grouped_forward(it.ctx, it.view_begin, it.view_count, it.I, it.IAbsorb, nullptr, b->cap_stream,
