@@ -2869,8 +2869,10 @@ constexpr int kCQ = 0, kCId = 3, kCKf = 6, kCKr = 7, kCE = 8, kCD = 11, kCG = 14
 // from the brick centre: for each staged pixel of rows [q0, q1] x columns
 // [w0, w1], the lattice samples between the ray's crossings of the cell's
 // planes X, X + 1 (and Y, Z), weighted into the eight corners, times the
-// pixel's dl/dL into acc[corner].  Per sample: three positions, three
-// complements, four (y, z) products and eight accumulations.
+// pixel's dl/dL into acc[corner].  Bound by VALU issue: a loop over the samples
+// (21 instructions each) ran as long as the lane with the most of them, so the
+// sum over a ray's samples is taken in closed form (~45 instructions): the
+// 3 x 256^3 gradient step 95.2 -> 90.0 ms.
 template <int M>
 __device__ __forceinline__ void cell_pixels(const float *rec0, int rs, int q0, int q1, int w0, int w1, float X,
                                             float Y, float Z, float ox, float oy, float oz, float Kf,
@@ -2891,37 +2893,30 @@ __device__ __forceinline__ void cell_pixels(const float *rec0, int rs, int q0, i
             if (k0 >= k1) continue;
             const float fX = rec[kCE + 0] - ox, fY = rec[kCE + 1] - oy, fZ = rec[kCE + 2] - oz;
             const float dX = rec[kCD + 0], dY = rec[kCD + 1], dZ = rec[kCD + 2];
+            // The corner weights summed over the n samples, in closed form
+            // about their midpoint: with T = t there, the samples at T + s d,
+            // s = -(n - 1) / 2 .. (n - 1) / 2, so sum s = sum s^3 = 0 and
+            // sum s^2 = n (n^2 - 1) / 12 = S.  A corner's weight is a product
+            // of A + s e per axis (A, e = T, d or 1 - T, -d), whose sum is
+            // n Ax Ay Az + S (Ax ey ez + ex (Ay ez + Az ey)).
+            const float n = (float)(k1 - k0);
+            const float S = n * fmaf(n, n, -1.0f) * (1.0f / 12.0f);
             // s = k - k*, from the brick's closest approach
-            float sj = (float)(k0 - __float_as_int(rec[kCKf])) - rec[kCKr];
+            const float sj = (float)(k0 - __float_as_int(rec[kCKf])) - rec[kCKr] + fmaf(0.5f, n, -0.5f);
+            const float tx = fmaf(sj, dX, fX), ty = fmaf(sj, dY, fY), tz = fmaf(sj, dZ, fZ);
+            const float ax = 1.0f - tx, ay = 1.0f - ty, az = 1.0f - tz;
+            const float nz0 = n * az, nz1 = n * tz, sY = S * dY, sZ = S * dZ, sYZ = sY * dZ;
+            const float y0z = ay * sZ, y1z = ty * sZ;
             float w[8];
-            {
-                // the first sample (k0 < k1) sets the weights
-                const float tx = fmaf(sj, dX, fX), ty = fmaf(sj, dY, fY), tz = fmaf(sj, dZ, fZ);
-                const float ax = 1.0f - tx, ay = 1.0f - ty, az = 1.0f - tz;
-                const float y0z0 = ay * az, y1z0 = ty * az, y0z1 = ay * tz, y1z1 = ty * tz;
-                w[0] = y0z0 * ax;
-                w[1] = y0z0 * tx;
-                w[2] = y1z0 * ax;
-                w[3] = y1z0 * tx;
-                w[4] = y0z1 * ax;
-                w[5] = y0z1 * tx;
-                w[6] = y1z1 * ax;
-                w[7] = y1z1 * tx;
-                sj += 1.0f;
-            }
-            for (int k = k0 + 1; k < k1; k++, sj += 1.0f) {
-                const float tx = fmaf(sj, dX, fX), ty = fmaf(sj, dY, fY), tz = fmaf(sj, dZ, fZ);
-                const float ax = 1.0f - tx, ay = 1.0f - ty, az = 1.0f - tz;
-                const float y0z0 = ay * az, y1z0 = ty * az, y0z1 = ay * tz, y1z1 = ty * tz;
-                w[0] = fmaf(y0z0, ax, w[0]);
-                w[1] = fmaf(y0z0, tx, w[1]);
-                w[2] = fmaf(y1z0, ax, w[2]);
-                w[3] = fmaf(y1z0, tx, w[3]);
-                w[4] = fmaf(y0z1, ax, w[4]);
-                w[5] = fmaf(y0z1, tx, w[5]);
-                w[6] = fmaf(y1z1, ax, w[6]);
-                w[7] = fmaf(y1z1, tx, w[7]);
-            }
+            auto pair = [&](int c, float B, float C) { // B: n Ay Az + S ey ez, C: S (Ay ez + Az ey)
+                const float q = dX * C;
+                w[c] = fmaf(B, ax, -q);
+                w[c + 1] = fmaf(B, tx, q);
+            };
+            pair(0, fmaf(ay, nz0, sYZ), -fmaf(az, sY, y0z));
+            pair(2, fmaf(ty, nz0, -sYZ), fmaf(az, sY, -y1z));
+            pair(4, fmaf(ay, nz1, -sYZ), fmaf(tz, -sY, y0z));
+            pair(6, fmaf(ty, nz1, sYZ), fmaf(tz, sY, y1z));
 #pragma unroll
             for (int m = 0; m < M; m++) {
                 const float g = rec[kCG + m];
